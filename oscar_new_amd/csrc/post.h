@@ -26,6 +26,7 @@ struct PostArgs {
   float* merged_lse;   // [rows] or null
   WindowArgs win;
   int64_t win_requests;  // min(n, max_reqs)
+  int32_t win_parts;     // window workgroups per request (window_parts)
   int32_t merge_wgs;     // workgroups of the merge role; the rest store windows
 };
 

@@ -53,6 +53,13 @@ __global__ __launch_bounds__(kThreads) void pre_attention_kernel(const PreArgs p
   rotate_rows16(a.query, a.qs0, a.qs1, p.hq_div, a.hq, p.q_rows, tile, p.rk_t, nullptr, p.qrot);
 }
 
+// Window workgroup w of a post-attention launch: part w % win_parts of one request's writers.
+__device__ __forceinline__ void window_role(const PostArgs& p, int w) {
+  const int req = w / p.win_parts, part = w - req * p.win_parts;
+  for (int head = 0; head < p.win.L.kv_heads; ++head)
+    store_window_request(p.win, req, head, part, p.win_parts);
+}
+
 // More than 16 splits. Workgroups [0, merge_wgs): R (token, query head) rows each (R = 4: a
 // scanned split merge per wavefront-row; R = 1: the four wavefronts merge the row together).
 // The remaining workgroups store the window of one request each; both branches have read the
@@ -76,8 +83,7 @@ __global__ __launch_bounds__(kThreads, 2) void post_attention_kernel(const PostA
     return;
   }
   if (blockIdx.y != 0) return;
-  const int req = static_cast<int>(blockIdx.x) - p.merge_wgs;
-  for (int head = 0; head < p.win.L.kv_heads; ++head) store_window_request(p.win, req, head);
+  window_role(p, static_cast<int>(blockIdx.x) - p.merge_wgs);
 }
 
 // Many rows (a long chunk: thousands of (token, query head) rows, one split): 16 rows per
@@ -99,7 +105,7 @@ post_attention_tile_kernel(const PostArgs p) {
   __shared__ GroupMergeLds group_lds;
   // The window-store workgroups come first: each walks its request's writers in sequence, so
   // started last they would end the launch.
-  const int64_t win = p.win_requests;
+  const int64_t win = p.win_requests * p.win_parts;
   if (static_cast<int64_t>(blockIdx.x) >= win) {
     const int64_t row0 = (static_cast<int64_t>(blockIdx.x) - win) * 16 * kTiles;
     const int64_t rows = p.rows;
@@ -108,8 +114,7 @@ post_attention_tile_kernel(const PostArgs p) {
         p.splits, s_h, s_l, &group_lds);
     return;
   }
-  const int req = static_cast<int>(blockIdx.x);
-  for (int head = 0; head < p.win.L.kv_heads; ++head) store_window_request(p.win, req, head);
+  window_role(p, static_cast<int>(blockIdx.x));
 }
 
 }  // namespace
@@ -451,6 +456,7 @@ int make_post_args(const float* history_partials, const float* history_lse, int3
   w.table_stride = table_stride;
   w.counts = counts;
   p.win_requests = n < max_reqs ? n : max_reqs;
+  p.win_parts = window_parts(n, p.win_requests, p.win_requests > 0 ? p.win_requests : 1, w.L, 256);
   return OSCAR_OK;
 }
 
@@ -478,9 +484,9 @@ extern "C" int oscar_post_attention(
     const bool two = mode == kMergeOneRound && splits == 1;  // 32 rows per workgroup
     const int64_t span = two ? 32 : 16;
     const int64_t tiles = (p.rows + span - 1) / span;
-    if (tiles + p.win_requests > 0x7fffffffll) return OSCAR_E_SHAPE;
+    if (tiles + p.win_requests * p.win_parts > 0x7fffffffll) return OSCAR_E_SHAPE;
     p.merge_wgs = static_cast<int32_t>(tiles);
-    const dim3 grid(static_cast<unsigned>(tiles + p.win_requests));
+    const dim3 grid(static_cast<unsigned>(tiles + p.win_requests * p.win_parts));
     if (two)
       hipLaunchKernelGGL((post_attention_tile_kernel<kMergeOneRound, 2>), grid, dim3(kThreads), 0,
                          s, p);
@@ -495,9 +501,9 @@ extern "C" int oscar_post_attention(
   const bool wide = mode != kMergeScanGroup && p.rows >= kPostWideFrom;
   const int rows_per_wg = mode == kMergeScanGroup ? 1 : wide ? kPostWideRows : kPostQuarterRows;
   const int64_t groups = (p.rows + rows_per_wg - 1) / rows_per_wg;
-  if (groups + p.win_requests > 0x7fffffffll) return OSCAR_E_SHAPE;
+  if (groups + p.win_requests * p.win_parts > 0x7fffffffll) return OSCAR_E_SHAPE;
   p.merge_wgs = static_cast<int32_t>(groups);
-  const dim3 grid(static_cast<unsigned>(groups + p.win_requests), wide ? 1 : 4);
+  const dim3 grid(static_cast<unsigned>(groups + p.win_requests * p.win_parts), wide ? 1 : 4);
   if (wide && mode == kMergeOneRound)
     hipLaunchKernelGGL((post_attention_kernel<kPostWideRows, kMergeOneRound, 4>), grid,
                        dim3(kThreads), 0, s, p);

@@ -37,9 +37,27 @@ struct WindowArgs {
 // Each index therefore has at most one writer. The writers are the sink tokens
 // [prefix, min(S, seq)) and the ring tokens [max(prefix, S, seq - C), seq): at most S + C of
 // them however long the chunk, taken kBatch at a time per wavefront (writer j by wavefront
-// (j / kBatch) mod 4), each batch's rows all requested before any is stored.
-__device__ __forceinline__ void store_window_request(const WindowArgs& a, int req, int head) {
-  constexpr int kBatch = 8;
+// (j / kBatch) mod (4 parts): wavefront w of the request's workgroup `part` of `parts`), each
+// batch's rows all requested before any is stored.
+constexpr int kWindowBatch = 8;
+constexpr int kWindowRound = (kThreads / kWave) * kWindowBatch;  // writers of a workgroup per round
+
+// Workgroups per (request, kv head). A workgroup's rounds of 32 writers follow one another, each
+// a round trip to memory (about 1.5 us), so a request with many writers (a prompt: up to S + C)
+// gets one workgroup per round while the launch stays under `cap` workgroups; decode steps
+// (at most n - requests + 1 tokens in one request) keep one. Four prompts of 4096 tokens,
+// S + C = 136: one workgroup each 20.6 us; nine of up to 1201, S + C = 324, two kv heads: 32.8 us.
+inline int window_parts(int64_t n, int64_t requests, int64_t groups, const Layout& L, int64_t cap) {
+  int64_t writers = n - requests + 1;
+  if (writers > L.sink + L.ring) writers = L.sink + L.ring;
+  int64_t parts = (writers + kWindowRound - 1) / kWindowRound;
+  if (parts > cap / groups) parts = cap / groups;
+  return static_cast<int>(parts < 1 ? 1 : parts);
+}
+
+__device__ __forceinline__ void store_window_request(const WindowArgs& a, int req, int head,
+                                                     int part = 0, int parts = 1) {
+  constexpr int kBatch = kWindowBatch;
   if (req >= a.counts[0]) return;
   const int qstart = a.qstarts[req];
   const int qend = min(a.qstarts[req + 1], a.counts[1]);
@@ -59,7 +77,7 @@ __device__ __forceinline__ void store_window_request(const WindowArgs& a, int re
                    reinterpret_cast<uintptr_t>(a.k) % 8 == 0 &&
                    reinterpret_cast<uintptr_t>(a.v) % 8 == 0;
   const bool vst = reinterpret_cast<uintptr_t>(a.window) % 8 == 0;
-  for (int base = wave * kBatch; base < total; base += (kThreads / kWave) * kBatch) {
+  for (int base = part * kWindowRound + wave * kBatch; base < total; base += parts * kWindowRound) {
     uint16_t kx[kBatch][4], vx[kBatch][4];
     int64_t dst[kBatch];
 #pragma unroll

@@ -3,15 +3,15 @@
 // Reference: oscar_ascend/kernels.py:544-620 (`_window_store_kernel`, `store_windows`).
 // Window index i < S holds position i. Ring index i >= S holds the LATEST position
 // pos < seq with pos = i - S (mod C); only current tokens (prefix <= pos < seq) are
-// written, so each ring slot has exactly one writer per step. One workgroup per
-// (request, kv head); wavefront w copies window indices w, w+4, ... (1 KiB each).
+// written, so each ring slot has exactly one writer per step. One workgroup per (request, kv
+// head, window_parts round of 32 writers).
 #include "window.h"
 
 namespace oscar {
 namespace {
 
 __global__ __launch_bounds__(kThreads) void store_windows_kernel(const WindowArgs a) {
-  store_window_request(a, blockIdx.x, blockIdx.y);
+  store_window_request(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
 }
 
 }  // namespace
@@ -49,8 +49,10 @@ extern "C" int oscar_store_windows(const void* key, int64_t k_s0, int64_t k_s1, 
   a.table = block_tables;
   a.table_stride = table_stride;
   a.counts = counts;
+  const int parts = window_parts(n, programs, programs * a.L.kv_heads, a.L, 2048);
   hipLaunchKernelGGL(store_windows_kernel,
-                     dim3(static_cast<unsigned>(programs), static_cast<unsigned>(a.L.kv_heads)),
+                     dim3(static_cast<unsigned>(programs), static_cast<unsigned>(a.L.kv_heads),
+                          static_cast<unsigned>(parts)),
                      dim3(kThreads), 0, as_stream(stream), a);
   return static_cast<int>(hipGetLastError());
 }

@@ -105,3 +105,41 @@ def test_window_bytes_match_oracle_through_ring_wraps_and_rollbacks():
             assert np.array_equal(bits(got_v).reshape(-1), want), \
                 f"fused step (one-launch post {one_launch}, layer step {layer}), step {index}"
         raw = fused  # the next step sees this step's INT2 slots and windows
+
+
+@pytest.mark.parametrize("lengths,max_reqs", [
+    ([32], 2),  # one round of 32 writers
+    ([33, 1], 3),  # one writer past a round
+    ([65, 700, 320], 4),  # more than S + C tokens: 11 rounds of the longest request
+    ([500, 333], 40),  # more request slots than requests
+    ([400], 300),  # fewer workgroups than rounds per request (post-attention: one)
+])
+def test_long_prompts_spread_over_workgroups_write_the_oracle_bytes(lengths, max_reqs):
+    # A request's writers go to several workgroups, 32 at a time (default sizes: S = 64,
+    # ring 260): the entry point and the layer step's post-attention launch.
+    cfg = OscarConfig()
+    layout, raw, _, _, meta, tables = make_state(lengths, [0] * len(lengths), cfg, kv_heads=H,
+                                                 max_reqs=max_reqs)
+    print(f"[windows] prompts {lengths} of {max_reqs} slots", flush=True)
+    n = _set_step(meta, tables, layout, [(0, length, 0) for length in lengths])
+    g = torch.Generator().manual_seed(19)
+    q = torch.randn(n, HQ, 256, generator=g).bfloat16().to(DEV)
+    k = torch.randn(n, H, 256, generator=g).bfloat16().to(DEV)
+    v = torch.randn(n, H, 256, generator=g).bfloat16().to(DEV)
+    want = O.store_windows(bits(native_views(raw, layout)[1]).reshape(-1), bits(k), bits(v),
+                           meta.query_start_loc.cpu().numpy(), meta.seq_lens.cpu().numpy(),
+                           tables.numpy(), meta.counts.cpu().numpy(), oracle_geometry(layout),
+                           meta.max_num_reqs)
+    eye = torch.eye(256, dtype=torch.bfloat16, device=DEV)
+    for fused in (False, True):
+        cache = raw.clone()
+        if fused:
+            impl = OscarAttentionImpl.standalone(HQ, 256, 1 / 16, H, cfg)
+            impl.set_rotations(eye, eye)
+            out = torch.empty(n, HQ * 256, dtype=torch.bfloat16, device=DEV)
+            impl.forward(None, q, k, v, native_views(cache, layout), meta, out)
+        else:
+            kernels.store_windows(k, v, layout.tensor_views(native_views(cache, layout))[1], meta,
+                                  layout)
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(native_views(cache, layout)[1]).reshape(-1), want), fused
