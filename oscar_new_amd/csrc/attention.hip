@@ -13,7 +13,10 @@ namespace {
 template <int RT>
 __global__ __launch_bounds__(kThreads) void raw_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[kRawSlots * kRawLdsPerSlot];
-  raw_block_staged<RT>(a, blockIdx.x, blockIdx.y, blockIdx.z, ring, kRawSlots);
+  if (RT == 1 && a.raw_waves)
+    raw_block_waves(a, blockIdx.x, blockIdx.y, blockIdx.z, ring);
+  else
+    raw_block_staged<RT>(a, blockIdx.x, blockIdx.y, blockIdx.z, ring, kRawSlots);
 }
 
 }  // namespace
@@ -98,6 +101,7 @@ int make_attn_args(const void* query, int64_t q_s0, int64_t q_s1, int64_t q_s2, 
   a.block_n = block_n;
   a.split_tokens = split_tokens;
   a.scale_log2 = scale * kLog2e;
+  a.raw_waves = raw_wave_form(qrows, max_query_len, programs * h);
   return OSCAR_OK;
 }
 

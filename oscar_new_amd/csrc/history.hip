@@ -1208,7 +1208,8 @@ static_assert(kDeviceUnitTasks * 4 <= kRingBytes, "the unit resolver's task list
 // kMode 5: as 3, and q rotation roles of the same launch (pre.h q_rotate_role) write the
 // rotated query into a.query: every wavefront requests its first chunks, then wavefront 3
 // waits for the roles' tile count and copies the task's rotated rows.
-template <int kMode>
+// kRawWaves (modes 3 to 5): the form of the BF16 role (raw_wave_form).
+template <int kMode, bool kRawWaves = false>
 __device__ __forceinline__ void history_pair_body(const AttnArgs& a, const FinishArgs* fin,
                                                   const LayerArgs* lay,
                                                   const PreArgs* pre = nullptr,
@@ -1234,12 +1235,16 @@ __device__ __forceinline__ void history_pair_body(const AttnArgs& a, const Finis
   static_assert(16 * kStageRowBytes + 4 * 2 * 8 * 16 * 4 <= 2 * kStageBytes,
                 "the layer step's 16-row staging tile and operand images fit wavefront 3's stages");
   static_assert(16 * kHeadDim * 2 <= kRingBytes, "the K/V store role's tile fits the ring");
+  static_assert(kRawWaveLds <= kRingBytes, "the BF16 role fits the ring");
   if constexpr (kMode == 3 || kMode == 4 || kMode == 5) {
     const int z = blockIdx.z;
     if (z < role_slices) {
       if (z == 0) {
-        raw_block_staged<1>(pre->attn, blockIdx.x, blockIdx.y, 0, s_ring,
-                            kRingBytes / kRawLdsPerSlot);
+        if constexpr (kRawWaves)
+          raw_block_waves(pre->attn, blockIdx.x, blockIdx.y, 0, s_ring);
+        else
+          raw_block_staged<1>(pre->attn, blockIdx.x, blockIdx.y, 0, s_ring,
+                              kRingBytes / kRawLdsPerSlot);
       } else {
         int r = ((z - 1) * static_cast<int>(gridDim.x) + static_cast<int>(blockIdx.x)) *
                     static_cast<int>(gridDim.y) + static_cast<int>(blockIdx.y);
@@ -1831,14 +1836,17 @@ struct HistoryPreArgs {
   int32_t role_slices;
 };
 
+template <bool kRawWaves>
 __global__ __launch_bounds__(kThreads, 2) void history_pre_kernel(const HistoryPreArgs h) {
-  history_pair_body<3>(h.a, nullptr, nullptr, &h.p, h.role_slices);
+  history_pair_body<3, kRawWaves>(h.a, nullptr, nullptr, &h.p, h.role_slices);
 }
+template <bool kRawWaves>
 __global__ __launch_bounds__(kThreads, 2) void history_pre_rot_kernel(const HistoryPreArgs h) {
-  history_pair_body<4>(h.a, nullptr, nullptr, &h.p, h.role_slices);
+  history_pair_body<4, kRawWaves>(h.a, nullptr, nullptr, &h.p, h.role_slices);
 }
+template <bool kRawWaves>
 __global__ __launch_bounds__(kThreads, 2) void history_pre_q_kernel(const HistoryPreArgs h) {
-  history_pair_body<5>(h.a, nullptr, nullptr, &h.p, h.role_slices);
+  history_pair_body<5, kRawWaves>(h.a, nullptr, nullptr, &h.p, h.role_slices);
   if (threadIdx.x == 0)
     q_sync_leave(h.p.qsync, static_cast<int>(gridDim.x * gridDim.y * gridDim.z));
 }
@@ -1896,12 +1904,12 @@ hipError_t launch_history_queue_pre(const AttnArgs& a, const PreArgs& p, int32_t
 hipError_t launch_history_pre(const AttnArgs& a, const PreArgs& p, int role_slices, dim3 grid,
                               bool rotate_query, hipStream_t stream) {
   const HistoryPreArgs h{a, p, role_slices};
-  if (p.qsync)
-    hipLaunchKernelGGL(history_pre_q_kernel, grid, dim3(kThreads), 0, stream, h);
-  else if (rotate_query)
-    hipLaunchKernelGGL(history_pre_rot_kernel, grid, dim3(kThreads), 0, stream, h);
-  else
-    hipLaunchKernelGGL(history_pre_kernel, grid, dim3(kThreads), 0, stream, h);
+  const bool waves = p.attn.raw_waves;
+  const auto kernel = p.qsync ? (waves ? history_pre_q_kernel<true> : history_pre_q_kernel<false>)
+                      : rotate_query
+                          ? (waves ? history_pre_rot_kernel<true> : history_pre_rot_kernel<false>)
+                          : (waves ? history_pre_kernel<true> : history_pre_kernel<false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, h);
   return hipGetLastError();
 }
 

@@ -592,5 +592,170 @@ __device__ __forceinline__ void raw_block_staged(const AttnArgs& a, int task, in
   }
   raw_finish<RT, kDirect>(a, s, head, split, st, n, g, wave);
 }
+// ---------------------------------------------------------------- decode form: blocks per wavefront
+
+// LDS of raw_block_waves: a 32-token block of K, then V rows per wavefront (later the merge
+// area), and the wavefronts' row maxima and sums behind them.
+constexpr int kRawWaveBlockBytes = kBlock * kHeadDim * 2;
+constexpr int kRawWaveRedBytes = 2 * 4 * 16 * 4;
+constexpr int kRawWaveLds = 4 * kRawWaveBlockBytes + kRawWaveRedBytes;
+
+// The rule of the entry points, from the query rows per task, the host bound on a request's
+// query tokens (0: unknown) and the (task, kv head) workgroups: few decode requests, whose
+// BF16 workgroups are the longest chains of the launch (one request of 700 tokens, 64 sink + 256
+// recent: history launch 19.9 -> 15.3 us, step 136 -> 118 us per four layers; of 100 k tokens
+// 150 -> 134). Longer requests keep the block-after-block form, whose bits the prefill and chunk
+// kernels reproduce; so do large batches (117 requests: 199 us against 196, the history stream
+// hides the chains) and tasks of more rows, whose work-queue launch has no registers left for
+// 256 accumulated dims (111 spilled: seven MTP requests 278 us against 267).
+constexpr int kRawWaveQueries = 16;
+constexpr int64_t kRawWaveWorkgroups = 64;
+inline bool raw_wave_form(int64_t qrows, int32_t max_query_len, int64_t workgroups) {
+  return qrows <= 8 && max_query_len >= 1 && max_query_len <= kRawWaveQueries &&
+         workgroups <= kRawWaveWorkgroups;
+}
+
+// The BF16 branch of a decode step with few requests: wavefront w takes the 32-token blocks w,
+// w + 4, ... of the split with its own online-softmax state for all 256 output dims, and the
+// four states are merged through LDS at the end: with the default window (11 blocks) three
+// rounds of memory latency and dependent MFMA chains instead of 11. A row with a single block
+// has the bits of raw_block_staged (the empty states add zeros), so a short request without
+// cached tokens still matches the prefill kernel. A wavefront's 16 KiB of LDS hold the block's K
+// rows (by DMA), then its V rows (requested into registers beside the K rows, the operand of P*V
+// takes one dim of eight tokens); K rows loaded straight into the A operands touch 64 lines per
+// instruction (117 requests 223 us). Every thread of the workgroup calls this; `lds` holds
+// kRawWaveLds bytes.
+__device__ __forceinline__ void raw_block_waves(const AttnArgs& a, int task, int head, int split,
+                                                uint8_t* lds) {
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  RawSetup<1> s;
+  if (!raw_setup<1, false>(a, task, head, split, n, g, s)) return;
+  State<1, 16> st;
+  state_init(st);
+  const int nblk = s.begin < s.end ? cdiv(s.end - s.begin, kBlock) : 0;
+  uint8_t* block = lds + wave * kRawWaveBlockBytes;
+  const uint32_t base = lds_addr(block);
+  raw_load_query(a, head, n, g, s);
+  // Lane l resolves raw index t0 + l % 32 of a block; the copies fetch their rows' pointers from
+  // it: copy i moves rows 2 i and 2 i + 1, 16 bytes per lane (whole rows, coalesced).
+  const int half_row = lane >> 5, piece = lane & 31;
+#pragma unroll 1
+  for (int b = wave; b < nblk; b += 4) {
+    const uint16_t *kp, *vp;
+    const int pos = raw_row(a, s.t, s.r, head, s.begin + kBlock * b + piece, s.end, kp, vp);
+    kp = kp ? kp : a.query;  // a row without a token: its score is masked, its P zero
+    vp = vp ? vp : a.query;
+    u32x4 vr[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      vr[i] = *reinterpret_cast<const u32x4*>(shfl_ptr(vp, 2 * i + half_row) + 8 * piece);
+    if (b != wave) OSCAR_WAIT_LGKM();  // every read of the previous block's V rows is done
+#pragma unroll 1
+    for (int i = 0; i < 16; i += 4) {  // K row r at 512 r, its piece p at p ^ (r % 8)
+      const uint16_t* src[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int row = 2 * (i + k) + half_row;
+        src[k] = shfl_ptr(kp, row) + 8 * (piece ^ (row & 7));
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) dma_dwordx4(src[k], base + 1024 * (i + k));
+    }
+    OSCAR_WAIT_VM(0);
+    f32x4 sc[1][2] = {{f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}};
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const u32x4 kd = *reinterpret_cast<const u32x4*>(
+            block + (16 * tt + n) * 512 + 16 * ((8 * g + m) ^ (n & 7)));
+        sc[0][tt] = mfma16x16x32(kd, s.qb[0][m], sc[0][tt]);
+      }
+    OSCAR_WAIT_LGKM();  // the K rows are read: the V rows take their place
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      *reinterpret_cast<u32x4*>(block + 1024 * i + 16 * lane) = vr[i];
+    bool live[8], ok[1][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int p = __shfl(pos, tau(g, e), kWave);
+      live[e] = p != 0x7fffffff;
+      ok[0][e] = live[e] && p <= s.t.prefix + s.qi_row[0];
+    }
+    u32x4 ap[1];
+    block_softmax(st, sc, ok, a.scale_log2, g, ap);
+    // Dims 16 n + 8 half + {0 .. 7} of the lane's eight tokens.
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      u32x4 vd[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const u32x4 x =
+            *reinterpret_cast<const u32x4*>(block + tau(g, e) * 512 + 32 * n + 16 * half);
+        vd[e] = live[e] ? x : u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        uint32_t vd2[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) vd2[e] = vd[e][j >> 1];
+        st.o[0][8 * half + j] = mfma16x16x32(ap[0], pv_operand(vd2, j), st.o[0][8 * half + j]);
+      }
+    }
+  }
+
+  // ---- merge of the four states: weights 2^(m_w - M), summed in wavefront order.
+  float* s_o = reinterpret_cast<float*>(lds);  // [wave][row][256]
+  float* s_red = reinterpret_cast<float*>(lds + 4 * kRawWaveBlockBytes);  // [max, sum][wave][row]
+  const float den_n = row_sum(st.psum[0]);
+  if (g == 0) {
+    s_red[wave * 16 + n] = st.m[0];
+    s_red[64 + wave * 16 + n] = den_n;
+  }
+  __syncthreads();  // every wavefront's V rows are read, too
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int row = 4 * g + v;
+    float mx = s_red[row];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) mx = fmaxf(mx, s_red[w * 16 + row]);
+    const float mw = s_red[wave * 16 + row];
+    const float f = mw == -INFINITY ? 0.f : exp2_hw(mw - mx);
+    float* dst = s_o + (wave * 16 + row) * kHeadDim + 16 * n;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<float4*>(dst + 4 * j) =
+          make_float4(st.o[0][4 * j][v] * f, st.o[0][4 * j + 1][v] * f, st.o[0][4 * j + 2][v] * f,
+                      st.o[0][4 * j + 3][v] * f);
+  }
+  __syncthreads();
+  const int row = threadIdx.x >> 4, d0 = 4 * (threadIdx.x & 15);
+  const RowInfo ri = row_info(a, s.t, head, row);
+  if (!ri.valid) return;
+  float mx = s_red[row];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) mx = fmaxf(mx, s_red[w * 16 + row]);
+  float sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float mw = s_red[w * 16 + row];
+    sum = fmaf(mw == -INFINITY ? 0.f : exp2_hw(mw - mx), s_red[64 + w * 16 + row], sum);
+  }
+  const float den = fmaxf(sum, 1.0e-30f);
+  const int64_t orow = (ri.token * a.hq + ri.qhead) * a.splits + split;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float* so = s_o + row * kHeadDim + d0 + 64 * q;
+    float r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      r[i] = (((so[i] + so[16 * kHeadDim + i]) + so[32 * kHeadDim + i]) + so[48 * kHeadDim + i]) / den;
+    *reinterpret_cast<float4*>(a.partials + orow * kHeadDim + d0 + 64 * q) =
+        make_float4(r[0], r[1], r[2], r[3]);
+  }
+  if ((threadIdx.x & 15) == 0) a.lse[orow] = row_lse(mx, sum);
+}
 
 }  // namespace oscar

@@ -41,7 +41,10 @@ __global__ __launch_bounds__(kThreads) void pre_attention_kernel(const PreArgs p
     // BF16 branch: workgroup (task, kv head), one split.
     const int h = a.L.kv_heads;
     const int task = bid / h, head = bid - task * h;
-    raw_block_staged<RT>(a, task, head, 0, smem, kRawSlots);
+    if (RT == 1 && a.raw_waves)
+      raw_block_waves(a, task, head, 0, smem);
+    else
+      raw_block_staged<RT>(a, task, head, 0, smem, kRawSlots);
     return;
   }
   if (bid < p.raw_wgs + p.kv_wgs) {
@@ -197,6 +200,7 @@ int make_pre_args(const void* query, int64_t q_s0, int64_t q_s1, const void* key
   a.splits = 1;
   a.block_n = block_n;
   a.scale_log2 = scale * kLog2e;
+  a.raw_waves = raw_wave_form(qrows, max_query_len, programs * h);
   p.rk_t = static_cast<const uint16_t*>(rk_t);
   p.rv_t = static_cast<const uint16_t*>(rv_t);
   p.qrot = static_cast<uint16_t*>(qrot);
