@@ -561,13 +561,17 @@ def history_rows(meta, layout, hq):
 
 def history_kernel_name(meta, layout, hq, tokens=0, split_tokens=0, use_queue=True):
     """The history-branch kernel ``attention_partials`` launches for ``tokens`` query rows:
-    the paired kernel up to 8 rows per task, the one-tile kernel up to 16, then the
-    two-row-group kernel (four wavefronts per workgroup up to 512 task rows, eight above), as
+    the paired kernel up to 8 rows per task; above, with more than 16 query tokens in some request
+    and the reference split rule, the 128-row-tile kernel of continuation chunks; the one-tile
+    kernel up to 16 rows, then the two-row-group kernel (four wavefronts per workgroup up to 512 task rows, eight above), as
     a work queue with token-bounded splits (``use_queue``, a grid of at most 2048 task
     rows)."""
     rows = history_rows(meta, layout, hq)
     if rows <= 8:
         return "history_pair_kernel"
+    mql = getattr(meta, "max_query_len", None)
+    if isinstance(mql, int) and mql > 16 and not split_tokens:
+        return "history_chunk_kernel"
     if rows <= 16:
         return "history_kernel<1>"
     programs = attention_programs(tokens, meta.max_num_reqs, layout.config.queries_per_tile)

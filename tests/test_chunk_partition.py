@@ -1,0 +1,48 @@
+"""Host side of the continuation-chunk history launch, on the CPU: the split counts, and the
+inline-asm copies of its kernel against the wait-state rule of the other kernels."""
+
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from oscar_new_amd.backend import OscarAttentionImpl
+from oscar_new_amd.config import OscarConfig, choose_chunk_splits
+from tests.test_isa_hazards import HIPCC, ROOT, _late_sites
+
+
+@pytest.mark.parametrize("tokens,requests,heads,q_heads,longest,want", [
+    (2048, 1, 1, 6, 34816, 5),  # 97 tiles: 485 of two rounds of 256 workgroups
+    (389, 1, 1, 6, 20400, 13),
+    (20, 1, 1, 6, 131072, 16),  # a tile or two: every split the one-round merge takes
+    (17, 1, 1, 6, 100, 1),  # a single pipeline step
+    (8192, 4, 2, 12, 2048, 1),  # tiles enough
+    (2048, 1, 1, 6, None, 1),  # no host-side length
+])
+def test_chunk_splits(tokens, requests, heads, q_heads, longest, want):
+    assert choose_chunk_splits(tokens, requests, heads, q_heads, longest) == want
+
+
+def test_long_chunks_take_the_chunk_splits():
+    from types import SimpleNamespace
+
+    meta = SimpleNamespace(num_reqs=1, num_actual_tokens=2048, max_query_len=2048, max_num_reqs=2,
+                           max_seq_len=34816, layout=None)
+    for policy, heads, want in (("device", 6, (5, 0)), ("mi355x", 6, (5, 0)),
+                                ("reference", 6, (1, 0)), ("device", 2, (1, 0))):
+        impl = OscarAttentionImpl.standalone(heads, 256, 1 / 16, 1, OscarConfig(),
+                                             split_policy=policy)
+        assert impl.partition_for(meta) == want
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="hipcc is not installed")
+def test_copies_keep_five_wait_states(tmp_path):
+    out = tmp_path / "history_chunk.s"
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17",
+                    "-fno-gpu-flush-denormals-to-zero", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", f"-I{ROOT / 'include'}", "--cuda-device-only", "-S",
+                    str(ROOT / "oscar_new_amd" / "csrc" / "history_chunk.hip"), "-o", str(out)],
+                   check=True, capture_output=True, timeout=600)
+    text = out.read_text()
+    assert text.count("global_load_lds_dword") >= 6
+    assert _late_sites(text) == []

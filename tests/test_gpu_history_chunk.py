@@ -1,0 +1,103 @@
+"""The history branch of continuation chunks (more than 16 query tokens per request: 128-row
+tiles sharing each chunk's operands) against the dequantized cache in float64, split by split:
+lengths around a tile's 128 rows and a chunk's 128 tokens, one and two KV heads, 4 to 8 query
+heads per KV head, several splits (some empty), requests of one token beside a chunk, a request
+cut short by the token count, and a history of more kernel blocks than one table.
+
+Bounds: the shared attention bounds (relative L2 1e-2, LSE 1e-2) for scores of unit spread."""
+
+import numpy as np
+import pytest
+import torch
+
+from oscar_new_amd import kernels
+from oscar_new_amd.config import OscarConfig
+from tests._state import assert_lse_close, assert_scaled_close, make_state, prepare_prefix
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _decoded(history, offsets):
+    """(K, V) float64 rows of the 160-byte records at `offsets`."""
+    rows = history[offsets[:, None] + torch.arange(160, device=DEV)]
+    out = []
+    for at in (0, 68):
+        data = rows[:, at : at + 64]
+        codes = torch.stack([data >> s & 3 for s in (0, 2, 4, 6)], -1).reshape(-1, 256).double()
+        sz = rows[:, at + 64 : at + 68].contiguous().view(torch.float16).double()
+        out.append(codes * sz[:, :1] + sz[:, 1:])
+    return out
+
+
+def _check(lengths, prefixes, splits, hq, kv_heads=1, sink=4, recent=128, pages=24, live=None):
+    cfg = OscarConfig(sink_tokens=sink, recent_tokens=recent)
+    torch.manual_seed(31)
+    layout, raw, hist, window, meta, tables = make_state(lengths, prefixes, cfg, pages=pages,
+                                                         kv_heads=kv_heads)
+    eye = torch.eye(256, dtype=torch.bfloat16, device=DEV)
+    ks = [torch.randn(n, kv_heads, 256).bfloat16() for n in lengths]
+    vs = [torch.randn(n, kv_heads, 256).bfloat16() for n in lengths]
+    prepare_prefix(ks, vs, eye, eye, hist, window, meta, tables, layout, prefixes)
+    n = sum(a - b for a, b in zip(lengths, prefixes))
+    q = torch.randn(n, hq, 256).bfloat16().to(DEV)
+    kernels.prepare_tasks(meta.query_start_loc, meta.counts, meta.tasks, meta.task_count,
+                          meta.max_num_reqs, cfg.queries_per_tile)
+    if live is not None:
+        meta.counts[1] = live
+    got, lse = kernels.attention_partials(q, None, None, hist, window, meta, layout, 1 / 16, splits,
+                                          raw=False)
+    torch.cuda.synchronize()
+    g, start = hq // kv_heads, 0
+    for r, (length, prefix) in enumerate(zip(lengths, prefixes)):
+        rows = slice(start, min(start + length - prefix, n if live is None else live))
+        start += length - prefix
+        prefix = length - (rows.stop - rows.start)  # as the kernels count a cut request's tokens
+        s = min(sink, prefix)
+        end = max(s, prefix - recent)
+        per = -(-(-(-(end - s) // cfg.block_n)) // splits) * cfg.block_n
+        slots = torch.tensor([int(tables[r, p // 128]) * 128 + p % 128 for p in range(s, end)],
+                             dtype=torch.int64, device=DEV)
+        for h in range(kv_heads):
+            page, within = slots // layout.physical_block_tokens, slots % layout.physical_block_tokens
+            k, v = _decoded(hist, page * layout.stripe_page_bytes + (within * kv_heads + h) * 160)
+            x = q[rows, h * g : h * g + g].double() / 16
+            for i in range(splits):
+                part = got[rows, h * g : h * g + g, i].cpu().numpy()
+                logs = lse[rows, h * g : h * g + g, i].cpu().numpy()
+                a, b = min(i * per, end - s), min((i + 1) * per, end - s)
+                if a == b:
+                    assert not part.any() and np.isneginf(logs).all()
+                    continue
+                score = x @ k[a:b].T
+                assert_scaled_close(part, (torch.softmax(score, -1) @ v[a:b]).cpu().numpy(),
+                                    f"request {r} head {h} split {i}")
+                assert_lse_close(logs, torch.logsumexp(score, -1).cpu().numpy(),
+                                 f"request {r} head {h} split {i} LSE")
+
+
+@pytest.mark.parametrize("lengths,prefixes,splits,hq,kv_heads", [
+    ([217], [200], 1, 6, 1),  # 17 query tokens, 68 history tokens: less than a tile or chunk
+    ([1044, 1043], [1023, 1022], 1, 6, 1),  # 126 rows: one tile
+    ([1300], [1278], 3, 6, 1),  # 132 rows: 4 rows in the second tile
+    ([388], [260], 2, 4, 1),  # exactly 128 history tokens, 512 rows
+    ([2000], [389], 4, 5, 1),  # tiles that split a query's five heads
+    ([1100, 700], [1000, 640], 2, 16, 2),  # two KV heads of eight
+    ([900, 2500, 40, 1700], [899, 2499, 0, 1500], 5, 6, 1),  # decodes, a first chunk, a chunk
+    ([3000], [2900], 16, 6, 1),
+    ([300], [150], 8, 6, 1),  # 18 history tokens: empty splits
+])
+def test_partials_against_the_dequantized_cache(lengths, prefixes, splits, hq, kv_heads):
+    print(f"[history chunk] {lengths} {prefixes} splits {splits} {hq}:{kv_heads}", flush=True)
+    _check(lengths, prefixes, splits, hq, kv_heads)
+
+
+def test_a_request_cut_short_by_the_token_count():
+    print("[history chunk] cut short", flush=True)
+    _check([900, 1300], [850, 1100], 2, 6, live=171)
+
+
+def test_more_history_blocks_than_the_table_holds():
+    # 2048 kernel blocks of 128 tokens lie in LDS; 280000 tokens in one split use 2188.
+    print("[history chunk] 280000 tokens", flush=True)
+    _check([280100], [280080], 1, 6, pages=368)
