@@ -124,6 +124,21 @@ int oscar_prepare_tasks(const int32_t* qstarts, const int32_t* counts, int32_t* 
                         int64_t copy_columns, void* stream);
 
 /*
+ * prepare_step -- no single reference entry point: the copies of a step's scheduler tensors
+ * into the fixed buffers (metadata.py:97-112) and prepare_tasks, one launch. Copies
+ * num_reqs + 1 query starts, num_reqs lengths, num_tokens slots and the first copy_columns
+ * table columns of each request, writes counts = {num_reqs, num_tokens} and the task table.
+ * Sources are contiguous (the table: rows of src_table_stride elements).
+ */
+int oscar_prepare_step(const int32_t* src_qstarts, const int32_t* src_seq_lens,
+                       const int64_t* src_slots, const int32_t* src_table,
+                       int64_t src_table_stride, int64_t copy_columns, int32_t num_reqs,
+                       int32_t num_tokens, int64_t max_reqs, int64_t max_tokens,
+                       int32_t query_tile, int32_t* qstarts, int32_t* seq_lens, int64_t* slots,
+                       int32_t* table, int64_t table_stride, int32_t* counts, int32_t* tasks,
+                       int32_t* task_count, int64_t task_capacity, void* stream);
+
+/*
  * attention_partials -- replaces kernels.py:439-482 `attention_partials(query, key,
  * value, history, window, meta, layout, scale, splits, raw)`.
  * Grid (programs, H, splits): program i serves task i if i < task_count[0]; `tasks` must

@@ -58,6 +58,8 @@ SIGNATURES = {
                                 POINTER(OscarLayout), POINTER(OscarClip), _P],
     "oscar_prepare_tasks": [_P, _P, _P, _P, _I64, _I64, _I32, _I64, _P, _I64, _P, _I64, _I64,
                             _P],
+    "oscar_prepare_step": [_P, _P, _P, _P, _I64, _I64, _I32, _I32, _I64, _I64, _I32, _P, _P, _P,
+                           _P, _I64, _P, _P, _P, _I64, _P],
     "oscar_attention_partials": [
         _P, _I64, _I64, _I64,  # query
         _P, _I64, _I64, _I64,  # key

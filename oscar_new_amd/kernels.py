@@ -18,6 +18,7 @@ from .config import CLIP_MODES, attention_programs
 __all__ = [
     "rotate",
     "store_int2",
+    "prepare_step",
     "prepare_tasks",
     "attention_partials",
     "merge_splits",
@@ -197,6 +198,48 @@ def prepare_tasks(qstarts, counts, tasks, task_count, max_reqs, query_tile, num_
             int(copy_columns) if source_table is not None else 0, _stream(qstarts),
         ),
         "prepare_tasks",
+    )
+
+
+def step_sources_fit(query_start_loc, seq_lens, slot_mapping, block_table, num_reqs, num_tokens,
+                     device):
+    """Whether ``prepare_step`` reads these scheduler tensors itself: contiguous rows of the
+    buffers' own types on the buffers' own device, at least as long as the step. Any other
+    form (other types, strides or devices) is left to tensor copies, which convert."""
+    return all(
+        t.dtype == dtype and t.dim() == 1 and t.shape[0] >= need and t.device == device
+        and t.stride(0) == 1
+        for t, dtype, need in ((query_start_loc, torch.int32, num_reqs + 1),
+                               (seq_lens, torch.int32, num_reqs),
+                               (slot_mapping, torch.int64, num_tokens))
+    ) and (block_table.dtype == torch.int32 and block_table.dim() == 2
+           and block_table.shape[0] >= num_reqs and block_table.device == device
+           and (block_table.shape[1] < 2 or block_table.stride(1) == 1)
+           and block_table.stride(0) >= block_table.shape[1])
+
+
+def prepare_step(query_start_loc, seq_lens, slot_mapping, block_table, num_reqs, num_tokens,
+                 copy_columns, qstarts, seqs, slots, table, counts, tasks, task_count, max_reqs,
+                 query_tile):
+    """One launch for a step's metadata: the copies of the scheduler's tensors into the fixed
+    buffers (``qstarts`` ... ``counts``) and ``prepare_tasks`` (reference metadata.py:97-112,
+    kernels.py:262-287). The sources must satisfy ``step_sources_fit``."""
+    sources = (query_start_loc, seq_lens, slot_mapping, block_table)
+    if not step_sources_fit(*sources, num_reqs, num_tokens, qstarts.device):
+        raise ValueError("prepare_step: the sources must be contiguous int32 / int64 tensors "
+                         "on the buffers' device, as long as the step")
+    if copy_columns > block_table.shape[1]:
+        raise ValueError("prepare_step: copy_columns exceeds the block table")
+    sources = [t.as_subclass(torch.Tensor) for t in sources]
+    _device_check(*sources, qstarts, seqs, slots, table, counts, tasks, task_count)
+    _ext.check(
+        _ext.library().oscar_prepare_step(
+            *(_ptr(t) for t in sources), sources[3].stride(0), int(copy_columns), int(num_reqs),
+            int(num_tokens), max_reqs, slots.shape[0], query_tile, _ptr(qstarts), _ptr(seqs),
+            _ptr(slots), _ptr(table), table.stride(0), _ptr(counts), _ptr(tasks),
+            _ptr(task_count), tasks.shape[0], _stream(qstarts),
+        ),
+        "prepare_step",
     )
 
 

@@ -2,9 +2,10 @@
 
 Reference: oscar_ascend/metadata.py:15-174. The builder is constructed by vLLM with
 ``(kv_cache_spec, layer_names, vllm_config, device)``, allocates its buffers once, and
-``build`` copies each step's scheduler metadata into them with asynchronous device copies
-(no host reads), then launches the task-table kernel, so a captured HIP graph replays with
-new lengths, pages and request counts. A capture (dummy) build clears ``counts``, which masks
+``build`` copies each step's scheduler metadata into them on the device (no host reads) and
+fills the task table, in one launch for tensors of the buffers' own types and as tensor copies
+and the task-table kernel otherwise, so a captured HIP graph replays with new lengths, pages
+and request counts. A capture (dummy) build clears ``counts``, which masks
 every cache access on the device. vLLM is not importable here: the builder is written against
 duck-typed vLLM objects, and ``OscarMetadataBuilder.standalone`` makes one without an engine.
 """
@@ -178,16 +179,21 @@ class OscarMetadataBuilder:
         dummy = in_dummy_run()
         max_seq_len = getattr(cm, "max_seq_len", None)
         copy_columns = 0
+        fused = False
         if dummy:
             # A capture run owns no pages, and vLLM invalidates its slot mapping after this
             # build: zero counts mask every cache access while every launch is recorded.
             self.counts.zero_()
         else:
-            self.qstarts[: nr + 1].copy_(cm.query_start_loc[: nr + 1], non_blocking=True)
-            self.seqs[:nr].copy_(cm.seq_lens[:nr], non_blocking=True)
-            self.slots[:nt].copy_(cm.slot_mapping[:nt], non_blocking=True)
-            self.counts[0].fill_(nr)
-            self.counts[1].fill_(nt)
+            sources = (cm.query_start_loc, cm.seq_lens, cm.slot_mapping, cm.block_table_tensor)
+            fused = self.counts.is_cuda and kernels.step_sources_fit(
+                *sources, nr, nt, self.counts.device)
+            if not fused:
+                self.qstarts[: nr + 1].copy_(cm.query_start_loc[: nr + 1], non_blocking=True)
+                self.seqs[:nr].copy_(cm.seq_lens[:nr], non_blocking=True)
+                self.slots[:nt].copy_(cm.slot_mapping[:nt], non_blocking=True)
+                self.counts[0].fill_(nr)
+                self.counts[1].fill_(nt)
             # Only the columns the longest request can reach (host-side bound) are copied.
             copy_columns = columns
             if isinstance(max_seq_len, int):
@@ -203,10 +209,16 @@ class OscarMetadataBuilder:
             if host is None or getattr(host, "device", None) is None or host.device.type != "cpu":
                 raise ValueError("query_start_loc_cpu must really be on CPU")
             query_ends = host[1 : nr + 1].tolist()
-        kernels.prepare_tasks(self.qstarts, self.counts, self.tasks, self.task_count,
-                              self.max_reqs, self.query_tile, num_reqs=1 if dummy else nr,
-                              source_table=cm.block_table_tensor, table=self.table,
-                              copy_columns=copy_columns)
+        if fused:
+            # One launch: the scheduler's tensors have the buffers' own types.
+            kernels.prepare_step(*sources, nr, nt, copy_columns, self.qstarts, self.seqs,
+                                 self.slots, self.table, self.counts, self.tasks,
+                                 self.task_count, self.max_reqs, self.query_tile)
+        else:
+            kernels.prepare_tasks(self.qstarts, self.counts, self.tasks, self.task_count,
+                                  self.max_reqs, self.query_tile, num_reqs=1 if dummy else nr,
+                                  source_table=cm.block_table_tensor, table=self.table,
+                                  copy_columns=copy_columns)
         seq_cpu = getattr(cm, "seq_lens_cpu", None)
         return OscarMetadata(
             self.qstarts, self.seqs, self.table, self.slots, self.counts, nr, nt,
