@@ -179,6 +179,25 @@ int oscar_attention_partials(const void* query, int64_t q_s0, int64_t q_s1, int6
                              float* lse, int32_t* queue_counters, void* stream);
 
 /*
+ * history_chunk -- the raw == 0 branch of attention_partials under the reference split rule
+ * (split_tokens 0), for continuation chunks: 128 consecutive (query, head) rows of a request per
+ * workgroup instead of one task row's. The same arguments, outputs and split ranges.
+ * max_reqs: upper bound on the requests that own task rows; it must not undercount (the grid is
+ * sized by it: oscar_history_chunk_tiles workgroups per kv head and split, for groups of
+ * `group` = hq / H query heads).
+ */
+int oscar_history_chunk(const void* query, int64_t q_s0, int64_t q_s1, int64_t q_s2,
+                        const void* history, int64_t history_bytes, const int32_t* qstarts,
+                        const int32_t* seq_lens, const int32_t* block_tables,
+                        int64_t table_stride, int64_t table_columns, const int32_t* counts,
+                        const int32_t* tasks, const int32_t* task_count, int64_t n, int64_t hq,
+                        int64_t programs, int64_t max_reqs, int32_t splits, int32_t block_n,
+                        int32_t query_tile, float scale, const oscar_layout* layout,
+                        float* partials, float* lse, void* stream);
+int64_t oscar_history_chunk_tiles(int64_t n, int64_t max_reqs, int64_t programs,
+                                  int32_t query_tile, int32_t group);
+
+/*
  * merge_splits -- replaces kernels.py:506-511 `merge_splits(partials, lse, counts)`.
  * out[t, q, :] = sum_s e^{lse_s - M} P_s / sum_s e^{lse_s - M} (bf16) and
  * logsum[t, q] = M + log(sum) or -inf; rows t >= counts[1] become 0 / -inf.

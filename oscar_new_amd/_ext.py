@@ -71,6 +71,13 @@ SIGNATURES = {
         _I32,  # split_tokens
         POINTER(OscarLayout), _P, _P, _P, _P,  # layout, partials, lse, queue counters, stream
     ],
+    "oscar_history_chunk": [
+        _P, _I64, _I64, _I64, _P, _I64,  # query, history
+        _P, _P, _P, _I64, _I64, _P, _P, _P,  # qstarts .. table columns, counts, tasks, count
+        _I64, _I64, _I64, _I64, _I32, _I32, _I32, _F,  # n hq programs max_reqs splits bn qt scale
+        POINTER(OscarLayout), _P, _P, _P,  # layout, partials, lse, stream
+    ],
+    "oscar_history_chunk_tiles": [_I64, _I64, _I64, _I32, _I32],
     "oscar_merge_splits": [_P, _P, _P, _I64, _I64, _I32, _I32, _P, _P, _P],
     "oscar_merge_paths": [_P, _P, _P, _P, _P, _I64, _I64, _I32, _P, _P, _P],
     "oscar_store_windows": [_P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _P,
@@ -177,7 +184,8 @@ SIGNATURES = {
     "oscar_calibration_workspace_bytes": [_I32, _I32],
     "oscar_calibrated_rotations": [_P, _I32, _I32, _I32, _F, _P, _I64, _P, _P, _P, _P],
 }
-RESTYPES = {"oscar_noalloc_scratch_bytes": c_int64, "oscar_calibration_workspace_bytes": c_int64}
+RESTYPES = {"oscar_noalloc_scratch_bytes": c_int64, "oscar_calibration_workspace_bytes": c_int64,
+            "oscar_history_chunk_tiles": c_int64}
 NOALLOC_SCRATCH_BYTES = 32 << 20  # OSCAR_NOALLOC_SCRATCH_BYTES
 
 _lib = None

@@ -345,11 +345,6 @@ __device__ __forceinline__ void write_unused_splits(const AttnArgs& a, const Tas
 hipError_t launch_history(const AttnArgs& a, dim3 grid, int rows, hipStream_t stream,
                           int32_t* queue = nullptr);
 
-// The history branch of continuation chunks (history_chunk.hip): more than kChunkQueries query
-// tokens per request, more than 8 query rows per task, the reference split rule.
-constexpr int32_t kChunkQueries = 16;
-hipError_t launch_history_chunk(const AttnArgs& a, int64_t programs, hipStream_t stream);
-
 // The checks and fields of one attention_partials launch (attention.hip): OSCAR_OK with *out
 // filled and *qrows = query rows per task, or the entry point's error code. Nothing is
 // launched when n == 0 (OSCAR_OK before the pointer checks).

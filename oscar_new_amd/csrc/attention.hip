@@ -137,8 +137,6 @@ extern "C" int oscar_attention_partials(
   const dim3 grid(static_cast<unsigned>(programs), static_cast<unsigned>(a.L.kv_heads),
                   static_cast<unsigned>(z));
   hipStream_t s = as_stream(stream);
-  if (!raw && qrows > 8 && max_query_len > kChunkQueries && split_tokens == 0)
-    return static_cast<int>(launch_history_chunk(a, programs, s));
   if (!raw)
     return static_cast<int>(launch_history(a, grid, static_cast<int>(qrows), s, queue_counters));
   if (qrows <= 16)

@@ -565,18 +565,46 @@ __global__ __launch_bounds__(kThreadsC, 2) void history_chunk_kernel(const AttnA
 
 }  // namespace
 
-hipError_t launch_history_chunk(const AttnArgs& a, int64_t programs, hipStream_t stream) {
-  // Tiles of all requests: at most one per 128 task rows and one more per request; `programs`
-  // task rows hold at most programs - ceil(n / query tile) + 1 requests (or one per token).
-  const int64_t full = (a.n + a.qt - 1) / a.qt;
-  const int64_t reqs = programs > full ? programs - full + 1 : 1;
-  int64_t tiles = programs * a.qt * a.g / kRowsC + (reqs < a.n ? reqs : a.n);
-  if (tiles > programs) tiles = programs;
-  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(a.L.kv_heads),
-                  static_cast<unsigned>(a.splits));
-  hipLaunchKernelGGL(history_chunk_kernel, grid, dim3(kThreadsC), 0, stream, a,
-                     static_cast<int32_t>(programs));
-  return hipGetLastError();
+// Grid x of the launch: at least the tiles find_tile can find. A request of q query tokens holds
+// ceil(q / qt) task rows of qt g <= 32 rows, x rows in all, and starts ceil(x / 128) <= (x + 127) /
+// 128 tiles; over at most `reqs` requests of n tokens and `programs` task rows, x sums to at most
+// the smaller of programs qt g and (n + (qt - 1) reqs) g. A task row starts at most one tile.
+int64_t history_chunk_tiles(int64_t n, int64_t max_reqs, int64_t programs, int64_t qt, int64_t g) {
+  const int64_t reqs = n < max_reqs ? n : max_reqs;
+  const int64_t by_tasks = programs * qt * g, by_tokens = (n + (qt - 1) * reqs) * g;
+  const int64_t rows = by_tasks < by_tokens ? by_tasks : by_tokens;
+  const int64_t tiles = (rows + (kRowsC - 1) * reqs) / kRowsC;
+  return tiles < programs ? tiles : programs;
 }
 
 }  // namespace oscar
+
+extern "C" int64_t oscar_history_chunk_tiles(int64_t n, int64_t max_reqs, int64_t programs,
+                                             int32_t query_tile, int32_t group) {
+  return oscar::history_chunk_tiles(n, max_reqs, programs, query_tile, group);
+}
+
+extern "C" int oscar_history_chunk(
+    const void* query, int64_t q_s0, int64_t q_s1, int64_t q_s2, const void* history,
+    int64_t history_bytes, const int32_t* qstarts, const int32_t* seq_lens,
+    const int32_t* block_tables, int64_t table_stride, int64_t table_columns,
+    const int32_t* counts, const int32_t* tasks, const int32_t* task_count, int64_t n, int64_t hq,
+    int64_t programs, int64_t max_reqs, int32_t splits, int32_t block_n, int32_t query_tile,
+    float scale, const oscar_layout* layout, float* partials, float* lse, void* stream) {
+  using namespace oscar;
+  if (max_reqs < 1 || max_reqs > 0x7fffffffll) return OSCAR_E_SHAPE;
+  AttnArgs a;
+  int64_t qrows = 0;
+  const int st = make_attn_args(query, q_s0, q_s1, q_s2, nullptr, 0, 0, 1, nullptr, 0, 0, 1,
+                                history, history_bytes, nullptr, 0, qstarts, seq_lens,
+                                block_tables, table_stride, table_columns, counts, tasks,
+                                task_count, n, hq, programs, splits, block_n, query_tile, 0, scale,
+                                0, 0, layout, partials, lse, &a, &qrows);
+  if (st != OSCAR_OK || n == 0) return st;
+  const int64_t tiles = history_chunk_tiles(n, max_reqs, programs, query_tile, a.g);
+  const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(a.L.kv_heads),
+                  static_cast<unsigned>(splits));
+  hipLaunchKernelGGL(history_chunk_kernel, grid, dim3(kThreadsC), 0, as_stream(stream), a,
+                     static_cast<int32_t>(programs));
+  return static_cast<int>(hipGetLastError());
+}

@@ -280,6 +280,21 @@ def attention_partials(query, key, value, history, window, meta, layout, scale, 
     table = _int32(meta.block_tables, "block_tables")
     max_query_len = getattr(meta, "max_query_len", None)
     max_query_len = int(max_query_len) if isinstance(max_query_len, int) else 0
+    if not raw and _chunk_history(meta, layout, hq, split_tokens):
+        _ext.check(
+            _ext.library().oscar_history_chunk(
+                _ptr(query), *query.stride(), _ptr(history),
+                history.numel() * history.element_size(),
+                _ptr(_int32(meta.query_start_loc, "query_start_loc")),
+                _ptr(_int32(meta.seq_lens, "seq_lens")), _ptr(table), table.stride(0),
+                table.shape[1], _ptr(_int32(meta.counts, "counts")),
+                _ptr(_int32(meta.tasks, "tasks")), _ptr(_int32(meta.task_count, "task_count")),
+                n, hq, programs, meta.max_num_reqs, splits, cfg.block_n, cfg.queries_per_tile,
+                float(scale), layout_struct(layout), _ptr(partials), _ptr(lse), _stream(query),
+            ),
+            "history_chunk",
+        )
+        return partials, lse
     kq = key if raw else None
     vq = value if raw else None
     _ext.check(
@@ -602,18 +617,25 @@ def history_rows(meta, layout, hq):
     return (mql if isinstance(mql, int) and 0 < mql < qt else qt) * (hq // layout.kv_heads)
 
 
+def _chunk_history(meta, layout, hq, split_tokens):
+    """Whether a history launch is the 128-row-tile kernel of continuation chunks: more than 16
+    query tokens in some request, more than 8 query rows per task, the reference split rule."""
+    mql = getattr(meta, "max_query_len", None)
+    return (isinstance(mql, int) and mql > 16 and not split_tokens
+            and history_rows(meta, layout, hq) > 8)
+
+
 def history_kernel_name(meta, layout, hq, tokens=0, split_tokens=0, use_queue=True):
     """The history-branch kernel ``attention_partials`` launches for ``tokens`` query rows:
     the paired kernel up to 8 rows per task; above, with more than 16 query tokens in some request
     and the reference split rule, the 128-row-tile kernel of continuation chunks; the one-tile
-    kernel up to 16 rows, then the two-row-group kernel (four wavefronts per workgroup up to 512 task rows, eight above), as
-    a work queue with token-bounded splits (``use_queue``, a grid of at most 2048 task
+    kernel up to 16 rows, then the two-row-group kernel (four wavefronts per workgroup up to 512
+    task rows, eight above), as a work queue with token-bounded splits (``use_queue``, a grid of at most 2048 task
     rows)."""
     rows = history_rows(meta, layout, hq)
     if rows <= 8:
         return "history_pair_kernel"
-    mql = getattr(meta, "max_query_len", None)
-    if isinstance(mql, int) and mql > 16 and not split_tokens:
+    if _chunk_history(meta, layout, hq, split_tokens):
         return "history_chunk_kernel"
     if rows <= 16:
         return "history_kernel<1>"

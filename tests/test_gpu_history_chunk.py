@@ -1,8 +1,10 @@
 """The history branch of continuation chunks (more than 16 query tokens per request: 128-row
 tiles sharing each chunk's operands) against the dequantized cache in float64, split by split:
 lengths around a tile's 128 rows and a chunk's 128 tokens, one and two KV heads, 4 to 8 query
-heads per KV head, several splits (some empty), requests of one token beside a chunk, a request
-cut short by the token count, and a history of more kernel blocks than one table.
+heads per KV head, several splits (some empty), requests of one token beside a chunk (also in
+batches whose task rows reach the token count, and with query tiles of 1 and 2), a request cut
+short by the token count, and a history of more chunks than one table. The output buffers hold NaN
+before the launch, so that a row that is not written fails.
 
 Bounds: the shared attention bounds (relative L2 1e-2, LSE 1e-2) for scores of unit spread."""
 
@@ -30,11 +32,12 @@ def _decoded(history, offsets):
     return out
 
 
-def _check(lengths, prefixes, splits, hq, kv_heads=1, sink=4, recent=128, pages=24, live=None):
-    cfg = OscarConfig(sink_tokens=sink, recent_tokens=recent)
+def _check(lengths, prefixes, splits, hq, kv_heads=1, sink=4, recent=128, pages=24, live=None,
+           query_tile=4, max_reqs=8):
+    cfg = OscarConfig(sink_tokens=sink, recent_tokens=recent, queries_per_tile=query_tile)
     torch.manual_seed(31)
     layout, raw, hist, window, meta, tables = make_state(lengths, prefixes, cfg, pages=pages,
-                                                         kv_heads=kv_heads)
+                                                         kv_heads=kv_heads, max_reqs=max_reqs)
     eye = torch.eye(256, dtype=torch.bfloat16, device=DEV)
     ks = [torch.randn(n, kv_heads, 256).bfloat16() for n in lengths]
     vs = [torch.randn(n, kv_heads, 256).bfloat16() for n in lengths]
@@ -45,8 +48,11 @@ def _check(lengths, prefixes, splits, hq, kv_heads=1, sink=4, recent=128, pages=
                           meta.max_num_reqs, cfg.queries_per_tile)
     if live is not None:
         meta.counts[1] = live
-    got, lse = kernels.attention_partials(q, None, None, hist, window, meta, layout, 1 / 16, splits,
-                                          raw=False)
+    assert kernels.history_kernel_name(meta, layout, hq) == "history_chunk_kernel"
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setattr(torch, "empty", lambda *a, **k: torch.full(*a, float("nan"), **k))
+        got, lse = kernels.attention_partials(q, None, None, hist, window, meta, layout, 1 / 16,
+                                              splits, raw=False)
     torch.cuda.synchronize()
     g, start = hq // kv_heads, 0
     for r, (length, prefix) in enumerate(zip(lengths, prefixes)):
@@ -90,6 +96,22 @@ def _check(lengths, prefixes, splits, hq, kv_heads=1, sink=4, recent=128, pages=
 def test_partials_against_the_dequantized_cache(lengths, prefixes, splits, hq, kv_heads):
     print(f"[history chunk] {lengths} {prefixes} splits {splits} {hq}:{kv_heads}", flush=True)
     _check(lengths, prefixes, splits, hq, kv_heads)
+
+
+@pytest.mark.parametrize("decodes,group,query_tile,max_reqs", [
+    (133, 4, 4, 257),  # 134 tiles; as many task rows as tokens
+    (250, 6, 4, 257),
+    (256, 5, 4, 257),  # every request slot in use
+    (26, 8, 2, 257),
+    (3, 16, 1, 257),
+    (5, 9, 1, 8),
+])
+def test_a_short_chunk_beside_many_decodes(decodes, group, query_tile, max_reqs):
+    print(f"[history chunk] {decodes} decodes group {group} tile {query_tile}", flush=True)
+    lengths = [210 + 7 * (i % 11) for i in range(decodes)] + [260]
+    prefixes = [n - 1 for n in lengths[:-1]] + [243]
+    _check(lengths, prefixes, 1, group, pages=decodes + 3, query_tile=query_tile,
+           max_reqs=max_reqs)
 
 
 def test_a_request_cut_short_by_the_token_count():
