@@ -677,7 +677,8 @@ def in_step_launch(impl, w, layers, splits, split_tokens):
         kernels.attention_partials(qrot, w.k, w.v, h, win, meta, layout, 1 / 16, splits, False,
                                    split_tokens=split_tokens)
 
-    return kernels.history_kernel_name(meta, layout, 6, ntok, split_tokens), hist, fn
+    return kernels.history_kernel_name(meta, layout, 6, ntok, split_tokens,
+                                       splits=splits), hist, fn
 
 
 def branch_launch(impl, w, layers, splits, split_tokens):
@@ -702,7 +703,8 @@ def branch_launch(impl, w, layers, splits, split_tokens):
         kernels.attention_partials(qrot, w.k, w.v, h, win, w.meta, w.layout, 1 / 16, splits,
                                    False, split_tokens=split_tokens)
 
-    return kernels.history_kernel_name(w.meta, w.layout, 6, ntok, split_tokens), hist, fn
+    return kernels.history_kernel_name(w.meta, w.layout, 6, ntok, split_tokens,
+                                       splits=splits), hist, fn
 
 
 def time_launch(fn, nlayers, steps, use_graph, stream=None, pool=None):

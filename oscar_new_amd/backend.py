@@ -24,8 +24,8 @@ import os
 import torch
 
 from . import kernels
-from .config import (OscarConfig, attention_programs, choose_chunk_splits,
-                     choose_device_partition, choose_history_partition, choose_splits)
+from .config import (OscarConfig, attention_programs, choose_chunk_splits, choose_device_partition,
+                     choose_history_partition, choose_splits, chunk_kernel_pays)
 
 SPLIT_POLICIES = ("device", "reference", "mi355x")
 ENV_SPLIT_POLICY = "OSCAR_AMD_SPLIT_POLICY"
@@ -270,14 +270,23 @@ class OscarAttentionImpl:
         policies leave the slots of the pre-attention role workgroups free when those share the
         history launch. The one-launch forms (``one_launch_post``, ``layer_step``) count a grid
         of split slots and take the "mi355x" partition under "device". Continuation chunks (more
-        than 16 query tokens in a request) take ``choose_chunk_splits`` under both."""
+        than 16 query tokens in a request) take ``choose_chunk_splits`` under both where the kernel
+        of those splits pays, and one split otherwise."""
         if self.split_policy == "reference":
             return choose_splits(meta.num_reqs, self.num_kv_heads, meta.max_query_len), 0
         group = self.num_heads // self.num_kv_heads
         if meta.max_query_len > 16 and self.cfg.queries_per_tile * group > 8:
-            return choose_chunk_splits(
-                int(meta.num_actual_tokens if tokens is None else tokens), meta.num_reqs,
-                self.num_kv_heads, self.num_heads, getattr(meta, "max_seq_len", None)), 0
+            n = int(meta.num_actual_tokens if tokens is None else tokens)
+            longest = getattr(meta, "max_seq_len", None)
+            longest = longest if isinstance(longest, int) else None
+            splits = choose_chunk_splits(n, meta.num_reqs, self.num_kv_heads, self.num_heads,
+                                         longest)
+            if not chunk_kernel_pays(n, meta.num_reqs, self.num_kv_heads, self.num_heads, splits,
+                                     longest, getattr(meta, "total_seq_len", None),
+                                     getattr(meta, "total_query_keys", None),
+                                     self.cfg.queries_per_tile):
+                splits = 1
+            return splits, 0
         roles = self._roles_share_history_launch(meta)
         if self.split_policy == "device" and not (self.one_launch_post or self.layer_step):
             n = int(meta.num_actual_tokens if tokens is None else tokens)

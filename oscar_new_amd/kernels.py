@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from . import _ext
-from .config import CLIP_MODES, attention_programs
+from .config import CLIP_MODES, attention_programs, chunk_kernel_pays
 
 __all__ = [
     "rotate",
@@ -244,7 +244,7 @@ def prepare_step(query_start_loc, seq_lens, slot_mapping, block_table, num_reqs,
 
 
 def attention_partials(query, key, value, history, window, meta, layout, scale, splits, raw,
-                       split_tokens=0, use_queue=True):
+                       split_tokens=0, use_queue=True, chunk=None):
     """Per-split partial attention and LSE of one branch (reference kernels.py:439-482).
 
     raw=False: INT2 history (``query`` must be the rotated query). raw=True: BF16 sink /
@@ -260,9 +260,14 @@ def attention_partials(query, key, value, history, window, meta, layout, scale, 
     ``use_queue`` (no reference counterpart): tasks of 17-32 rows with token-bounded splits
     run as a work queue over the units in use (``queue_counters``); the same bits as the
     grid form (``use_queue=False``).
+    ``chunk`` (history branch under the reference split rule; no reference counterpart): the
+    128-row-tile kernel of continuation chunks, within rounding of the others; by default where
+    the metadata's host-side lengths say that it pays (``config.chunk_kernel_pays``).
     """
     if raw and split_tokens:
         raise ValueError("split_tokens applies to the history branch only")
+    if chunk and (raw or split_tokens):
+        raise ValueError("chunk applies to the history branch under the reference split rule")
     _device_check(query, key, value, history, window)
     n, hq, d = query.shape
     cfg = layout.config
@@ -280,7 +285,8 @@ def attention_partials(query, key, value, history, window, meta, layout, scale, 
     table = _int32(meta.block_tables, "block_tables")
     max_query_len = getattr(meta, "max_query_len", None)
     max_query_len = int(max_query_len) if isinstance(max_query_len, int) else 0
-    if not raw and _chunk_history(meta, layout, hq, split_tokens):
+    if chunk or (not raw and chunk is None
+                 and _chunk_history(meta, layout, hq, n, splits, split_tokens)):
         _ext.check(
             _ext.library().oscar_history_chunk(
                 _ptr(query), *query.stride(), _ptr(history),
@@ -617,25 +623,31 @@ def history_rows(meta, layout, hq):
     return (mql if isinstance(mql, int) and 0 < mql < qt else qt) * (hq // layout.kv_heads)
 
 
-def _chunk_history(meta, layout, hq, split_tokens):
+def _chunk_history(meta, layout, hq, tokens, splits, split_tokens):
     """Whether a history launch is the 128-row-tile kernel of continuation chunks: more than 16
-    query tokens in some request, more than 8 query rows per task, the reference split rule."""
+    query tokens in some request, more than 8 query rows per task, the reference split rule, and
+    ``chunk_kernel_pays`` by the metadata's host-side request count and lengths."""
     mql = getattr(meta, "max_query_len", None)
-    return (isinstance(mql, int) and mql > 16 and not split_tokens
-            and history_rows(meta, layout, hq) > 8)
+    longest = getattr(meta, "max_seq_len", None)
+    return (isinstance(mql, int) and mql > 16 and not split_tokens and isinstance(longest, int)
+            and history_rows(meta, layout, hq) > 8
+            and chunk_kernel_pays(tokens, getattr(meta, "num_reqs", meta.max_num_reqs),
+                                  layout.kv_heads, hq, splits, longest,
+                                  getattr(meta, "total_seq_len", None),
+                                  getattr(meta, "total_query_keys", None),
+                                  layout.config.queries_per_tile))
 
 
-def history_kernel_name(meta, layout, hq, tokens=0, split_tokens=0, use_queue=True):
+def history_kernel_name(meta, layout, hq, tokens=0, split_tokens=0, use_queue=True, splits=1):
     """The history-branch kernel ``attention_partials`` launches for ``tokens`` query rows:
-    the paired kernel up to 8 rows per task; above, with more than 16 query tokens in some request
-    and the reference split rule, the 128-row-tile kernel of continuation chunks; the one-tile
-    kernel up to 16 rows, then the two-row-group kernel (four wavefronts per workgroup up to 512
+    the paired kernel up to 8 rows per task; above, the 128-row-tile kernel of continuation chunks
+    where it pays (``splits``: the launch's split count); the one-tile kernel up to 16 rows, then the two-row-group kernel (four wavefronts per workgroup up to 512
     task rows, eight above), as a work queue with token-bounded splits (``use_queue``, a grid of at most 2048 task
     rows)."""
     rows = history_rows(meta, layout, hq)
     if rows <= 8:
         return "history_pair_kernel"
-    if _chunk_history(meta, layout, hq, split_tokens):
+    if _chunk_history(meta, layout, hq, tokens, splits, split_tokens):
         return "history_chunk_kernel"
     if rows <= 16:
         return "history_kernel<1>"

@@ -47,6 +47,7 @@ class OscarMetadata:
     task_count: torch.Tensor | None = None
     max_seq_len: int | None = None  # host upper bound on seq_lens
     total_seq_len: int | None = None  # host sum of seq_lens
+    total_query_keys: int | None = None  # host sum of query tokens x seq_lens (chunks)
     merged_lse: torch.Tensor | None = None  # optional [n, hq] output of the merged LSE
     finish_counters: torch.Tensor | None = None  # zeroed int32 slots of one-launch post
     queue_counters: torch.Tensor | None = None  # two zeroed int32 work-queue counters
@@ -220,6 +221,13 @@ class OscarMetadataBuilder:
                                   source_table=cm.block_table_tensor, table=self.table,
                                   copy_columns=copy_columns)
         seq_cpu = getattr(cm, "seq_lens_cpu", None)
+        starts_cpu = getattr(cm, "query_start_loc_cpu", None)
+        total_query_keys = None
+        if not dummy and nr > 1 and cm.max_query_len > 16 and all(
+                isinstance(t, torch.Tensor) and t.device.type == "cpu" for t in (seq_cpu, starts_cpu)):
+            starts = starts_cpu.numpy()[: nr + 1]
+            total_query_keys = int(((starts[1:] - starts[:-1]).astype("int64")
+                                    * seq_cpu.numpy()[:nr]).sum())
         return OscarMetadata(
             self.qstarts, self.seqs, self.table, self.slots, self.counts, nr, nt,
             cm.max_query_len, self.max_reqs, self.layout, attn_state=state,
@@ -228,6 +236,7 @@ class OscarMetadataBuilder:
             task_count=self.task_count, max_seq_len=max_seq_len,
             finish_counters=self.finish_counters, queue_counters=self.queue_counters,
             total_seq_len=None if dummy or seq_cpu is None else int(seq_cpu[:nr].sum()),
+            total_query_keys=total_query_keys,
         )
 
     def build_for_cudagraph_capture(self, common_attn_metadata, attn_state="DecodeOnly"):

@@ -7,9 +7,11 @@ from pathlib import Path
 
 import pytest
 
-from oscar_new_amd import _ext
+from oscar_new_amd import _ext, kernels
 from oscar_new_amd.backend import OscarAttentionImpl
-from oscar_new_amd.config import OscarConfig, attention_programs, choose_chunk_splits
+from oscar_new_amd.config import (OscarConfig, attention_programs, choose_chunk_splits,
+                                  chunk_kernel_pays)
+from oscar_new_amd.layout import CacheLayout
 from tests.test_isa_hazards import HIPCC, ROOT, _late_sites
 
 
@@ -35,6 +37,69 @@ def test_long_chunks_take_the_chunk_splits():
         impl = OscarAttentionImpl.standalone(heads, 256, 1 / 16, 1, OscarConfig(),
                                              split_policy=policy)
         assert impl.partition_for(meta) == want
+
+
+# Steps that were measured with both kernels, on both sides of the rule (layer step in us with the
+# splits of choose_chunk_splits, and with the task-shaped kernel and one split).
+@pytest.mark.parametrize("tokens,requests,group,heads,longest,total,pairs,tiles", [
+    (2048, 1, 6, 1, 34816, None, None, True),  # 625, 810
+    (94, 31, 6, 1, 16064, 218000, 1230000, True),  # 30 decodes: 150, 258
+    (94, 31, 6, 1, 16064, 218000, None, True),
+    (314, 251, 6, 1, 16064, 1700000, 2710000, False),  # 250 decodes: 370, 302
+    (314, 251, 6, 1, 16064, None, None, False),
+    (267, 251, 6, 1, 4017, 425000, 490000, False),  # 154, 109
+    (124, 61, 4, 2, 16064, 420000, 1430000, False),  # 313, 183
+    (300, 1, 6, 1, 800, 800, None, False),  # 112, 101
+    (8192, 1, 6, 1, 24192, None, None, True),  # 1383, 1789
+    (2078, 31, 6, 1, 10048, 111000, 20679000, True),  # 341, 436
+    (404, 16, 6, 1, 20400, 117000, 8020000, True),
+])
+def test_steps_take_the_kernel_that_measured_faster(tokens, requests, group, heads, longest, total,
+                                                    pairs, tiles):
+    from types import SimpleNamespace
+
+    cfg = OscarConfig()
+    layout = CacheLayout(768, kv_heads=heads, config=cfg)
+    meta = SimpleNamespace(num_reqs=requests, num_actual_tokens=tokens, max_query_len=64,
+                           max_num_reqs=257, max_seq_len=longest, total_seq_len=total,
+                           total_query_keys=pairs, layout=layout)
+    impl = OscarAttentionImpl.standalone(group * heads, 256, 1 / 16, heads, cfg)
+    splits, split_tokens = impl.partition_for(meta)
+    name = kernels.history_kernel_name(meta, layout, group * heads, tokens, split_tokens,
+                                       splits=splits)
+    assert split_tokens == 0 and (name == "history_chunk_kernel") == tiles
+    assert tiles or splits == 1
+    # One split of a lone chunk leaves most CUs without a tile: the task-shaped kernel.
+    assert kernels.history_kernel_name(meta, layout, group * heads, tokens) == (
+        "history_chunk_kernel" if tokens == 8192 else
+        "history_kernel<1>" if group == 4 else "history_w8_kernel")
+
+
+def test_builder_sums_the_query_keys_of_chunk_steps(monkeypatch):
+    from types import SimpleNamespace
+
+    import torch
+
+    from oscar_new_amd.metadata import OscarMetadataBuilder
+
+    builder = OscarMetadataBuilder.standalone(CacheLayout(768, config=OscarConfig()), 4, 64, 4096,
+                                              "cpu")
+    monkeypatch.setattr(kernels, "prepare_tasks", lambda *a, **k: None)
+    for lengths, tokens, want in (([900, 40000, 30], [1, 20, 3], 900 + 800000 + 90),
+                                  ([900, 40000], [1, 4], None), ([500], [20], None)):
+        starts = torch.tensor([0] + tokens).cumsum(0).to(torch.int32)
+        lens = torch.tensor(lengths, dtype=torch.int32)
+        meta = builder.build(0, SimpleNamespace(
+            num_reqs=len(tokens), num_actual_tokens=sum(tokens), max_query_len=max(tokens),
+            query_start_loc=starts, query_start_loc_cpu=starts, seq_lens=lens, seq_lens_cpu=lens,
+            block_table_tensor=torch.zeros(len(tokens), 8, dtype=torch.int32),
+            slot_mapping=torch.zeros(sum(tokens), dtype=torch.int64)))
+        assert meta.total_query_keys == want
+
+
+def test_no_host_side_length_keeps_the_task_shaped_kernel():
+    assert not chunk_kernel_pays(2048, 1, 1, 6, 1, None)
+    assert chunk_kernel_pays(2048, 1, 1, 6, 5, 34816)
 
 
 def _tiles(lengths, query_tile, group):

@@ -48,11 +48,10 @@ def _check(lengths, prefixes, splits, hq, kv_heads=1, sink=4, recent=128, pages=
                           meta.max_num_reqs, cfg.queries_per_tile)
     if live is not None:
         meta.counts[1] = live
-    assert kernels.history_kernel_name(meta, layout, hq) == "history_chunk_kernel"
     with pytest.MonkeyPatch.context() as patch:
         patch.setattr(torch, "empty", lambda *a, **k: torch.full(*a, float("nan"), **k))
         got, lse = kernels.attention_partials(q, None, None, hist, window, meta, layout, 1 / 16,
-                                              splits, raw=False)
+                                              splits, raw=False, chunk=True)
     torch.cuda.synchronize()
     g, start = hq // kv_heads, 0
     for r, (length, prefix) in enumerate(zip(lengths, prefixes)):
