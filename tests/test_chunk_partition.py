@@ -22,6 +22,10 @@ from tests.test_isa_hazards import HIPCC, ROOT, _late_sites
     (17, 1, 1, 6, 100, 1),  # a single pipeline step
     (8192, 4, 2, 12, 2048, 1),  # tiles enough
     (2048, 1, 1, 6, None, 1),  # no host-side length
+    (8192, 1, 2, 12, 131072, 1),  # 128 MiB of split rows: a second split would pass it
+    (8192, 1, 1, 6, 24192, 1),  # a third split would pass it
+    (16384, 1, 1, 6, 262144, 1),
+    (16384, 1, 4, 32, 262144, 1),  # one split alone passes it
 ])
 def test_chunk_splits(tokens, requests, heads, q_heads, longest, want):
     assert choose_chunk_splits(tokens, requests, heads, q_heads, longest) == want
