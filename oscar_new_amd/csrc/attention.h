@@ -47,8 +47,6 @@ struct AttnArgs {
   // [n][hq][256] and, when non-null, their LSE [n][hq].
   uint16_t* direct_out;
   float* direct_lse;
-  // BF16 branch with its blocks spread over the workgroup's wavefronts (raw_block_waves).
-  bool raw_waves;
 };
 
 struct Task {

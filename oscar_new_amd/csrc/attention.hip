@@ -10,10 +10,10 @@
 namespace oscar {
 namespace {
 
-template <int RT>
+template <int RT, bool kRawWaves = false>
 __global__ __launch_bounds__(kThreads) void raw_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[kRawSlots * kRawLdsPerSlot];
-  if (RT == 1 && a.raw_waves)
+  if constexpr (kRawWaves)
     raw_block_waves(a, blockIdx.x, blockIdx.y, blockIdx.z, ring);
   else
     raw_block_staged<RT>(a, blockIdx.x, blockIdx.y, blockIdx.z, ring, kRawSlots);
@@ -101,7 +101,6 @@ int make_attn_args(const void* query, int64_t q_s0, int64_t q_s1, int64_t q_s2, 
   a.block_n = block_n;
   a.split_tokens = split_tokens;
   a.scale_log2 = scale * kLog2e;
-  a.raw_waves = raw_wave_form(qrows, max_query_len, programs * h);
   return OSCAR_OK;
 }
 
@@ -139,7 +138,9 @@ extern "C" int oscar_attention_partials(
   hipStream_t s = as_stream(stream);
   if (!raw)
     return static_cast<int>(launch_history(a, grid, static_cast<int>(qrows), s, queue_counters));
-  if (qrows <= 16)
+  if (raw_wave_form(qrows, max_query_len, programs * a.L.kv_heads))
+    hipLaunchKernelGGL((raw_kernel<1, true>), grid, dim3(kThreads), 0, s, a);
+  else if (qrows <= 16)
     hipLaunchKernelGGL(raw_kernel<1>, grid, dim3(kThreads), 0, s, a);
   else
     hipLaunchKernelGGL(raw_kernel<2>, grid, dim3(kThreads), 0, s, a);

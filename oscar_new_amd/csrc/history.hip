@@ -1824,13 +1824,12 @@ hipError_t launch_history_queue_pre(const AttnArgs& a, const PreArgs& p, int32_t
 }
 
 hipError_t launch_history_pre(const AttnArgs& a, const PreArgs& p, int role_slices, dim3 grid,
-                              bool rotate_query, hipStream_t stream) {
+                              bool rotate_query, bool raw_waves, hipStream_t stream) {
   const HistoryPreArgs h{a, p, role_slices};
-  const bool waves = p.attn.raw_waves;
-  const auto kernel = p.qsync ? (waves ? history_pre_q_kernel<true> : history_pre_q_kernel<false>)
+  const auto kernel = p.qsync ? (raw_waves ? history_pre_q_kernel<true> : history_pre_q_kernel<false>)
                       : rotate_query
-                          ? (waves ? history_pre_rot_kernel<true> : history_pre_rot_kernel<false>)
-                          : (waves ? history_pre_kernel<true> : history_pre_kernel<false>);
+                          ? (raw_waves ? history_pre_rot_kernel<true> : history_pre_rot_kernel<false>)
+                          : (raw_waves ? history_pre_kernel<true> : history_pre_kernel<false>);
   hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, h);
   return hipGetLastError();
 }

@@ -154,8 +154,9 @@ constexpr int kQSyncPolls = 4096;
 // role_slices + splits); z-slice 0 runs the BF16 branch of (task, kv head) (lean form, one
 // split), z-slices 1 .. role_slices - 1 the K/V store quads, the rest the history splits.
 // rotate_query: a.query is the unrotated query and each history workgroup rotates its rows.
+// raw_waves: the form of the BF16 branch (raw_wave_form).
 hipError_t launch_history_pre(const AttnArgs& a, const PreArgs& p, int role_slices, dim3 grid,
-                              bool rotate_query, hipStream_t stream);
+                              bool rotate_query, bool raw_waves, hipStream_t stream);
 
 // Task rows of a four-wavefront history work queue (its task lists fit 80 KB of LDS with the
 // unit's ring, two workgroups per CU).

@@ -604,6 +604,7 @@ __device__ __forceinline__ void raw_block_staged(const AttnArgs& a, int task, in
 constexpr int kRawWaveBlockBytes = kBlock * kHeadDim * 2;
 constexpr int kRawWaveRedBytes = 2 * 4 * 16 * 4;
 constexpr int kRawWaveLds = 4 * kRawWaveBlockBytes + kRawWaveRedBytes;
+static_assert(kRawWaveLds <= kRawSlots * kRawLdsPerSlot, "the staged form's LDS holds it");
 
 // The rule of the entry points, from the query rows per task, the host bound on a request's
 // query tokens (0: unknown) and the (task, kv head) workgroups: few decode requests, whose
