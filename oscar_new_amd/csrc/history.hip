@@ -1019,7 +1019,8 @@ __device__ __forceinline__ void history_queue_body(const AttnArgs& a, int32_t* c
         if (u < bf) {
           const int r = static_cast<int>(u);
           const int th = r >> 1;  // (task, kv head) as in the pre-attention launch
-          raw_block_staged<1>(pre->attn, th / heads, th % heads, 0, role_lds, 2, 16 * (r & 1));
+          raw_block_staged<1, false, true>(pre->attn, th / heads, th % heads, 0, role_lds, 2,
+                                           16 * (r & 1));
         } else {
           kv_store_role(*pre, static_cast<int>(u - bf - hist_units), role_lds);
         }

@@ -125,7 +125,11 @@ __device__ __forceinline__ void update_max(State<RT, kTiles>& st, const float (&
 }
 
 // p = 2^(s - m), the lane's sum and the bf16 P operand (lane (n, g): row n, tokens tau(g, e)).
-template <int RT, int kTiles>
+// kPerScore: the select of masked scores one by one, the same bits. The work queue's role takes it:
+// beside the history kernel's registers the row select costs 30 more reloads of spilled scalars
+// (64 ragged MTP requests 120.3 us per layer, with this form 118.8; 32 of 2000 to 8000 tokens 61.0
+// and 61.4, the other way round).
+template <bool kPerScore = false, int RT, int kTiles>
 __device__ __forceinline__ void block_p(State<RT, kTiles>& st, const float (&s2)[RT][8],
                                         u32x4 (&ap)[RT]) {
 #pragma unroll
@@ -138,7 +142,10 @@ __device__ __forceinline__ void block_p(State<RT, kTiles>& st, const float (&s2)
     float p[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      p[e] = exp2_hw(s2[rt][e] - m);
+      if constexpr (kPerScore)
+        p[e] = s2[rt][e] == -INFINITY ? 0.f : exp2_hw(s2[rt][e] - st.m[rt]);
+      else
+        p[e] = exp2_hw(s2[rt][e] - m);
       st.psum[rt] += p[e];
     }
 #pragma unroll
@@ -148,14 +155,14 @@ __device__ __forceinline__ void block_p(State<RT, kTiles>& st, const float (&s2)
 
 // The block's scores of row tile rt to log2 units with the causal / range mask, then the
 // lazy max, p, the lane's sum and the bf16 P operand.
-template <int RT, int kTiles>
+template <bool kPerScore = false, int RT, int kTiles>
 __device__ __forceinline__ void block_softmax(State<RT, kTiles>& st, const f32x4 (&sc)[RT][2],
                                               const bool (&ok)[RT][8], float scale_log2, int g,
                                               u32x4 (&ap)[RT]) {
   float s2[RT][8];
   block_scores(sc, ok, scale_log2, s2);
   update_max(st, s2, g);
-  block_p(st, s2, ap);
+  block_p<kPerScore>(st, s2, ap);
 }
 
 // B operand of P*V for output dim 16 n + j: the bf16 values of dim j of this lane's eight
@@ -344,7 +351,7 @@ __device__ __forceinline__ bool raw_setup(const AttnArgs& a, int task, int head,
 
 // Everything of a block after its scores: causal / range mask, online softmax, P*V into the
 // wavefront's 4 output tiles (dims 16 n + 4 w + jj).
-template <int RT>
+template <bool kPerScore = false, int RT>
 __device__ __forceinline__ void raw_block_tail(State<RT, 4>& st, const f32x4 (&sc)[RT][2],
                                                const RawSetup<RT>& s, const uint2 (&vq)[8],
                                                const int (&pos)[8], const bool (&live)[8],
@@ -355,7 +362,7 @@ __device__ __forceinline__ void raw_block_tail(State<RT, 4>& st, const f32x4 (&s
 #pragma unroll
     for (int e = 0; e < 8; ++e) ok[rt][e] = live[e] && pos[e] <= s.t.prefix + s.qi_row[rt];
   u32x4 ap[RT];
-  block_softmax(st, sc, ok, scale_log2, g, ap);
+  block_softmax<kPerScore>(st, sc, ok, scale_log2, g, ap);
 #pragma unroll
   for (int jj = 0; jj < 4; ++jj) {
     uint32_t vd2[8];
@@ -523,7 +530,7 @@ __device__ __forceinline__ void raw_wait_blocks(int ahead) {
 // workgroup calls this; `lds` holds slots x kRawLdsPerSlot bytes. `row0`: the task's first row
 // of the workgroup's RT row tiles (a task of more rows can be served 16 rows at a time: a row's
 // bits do not depend on the rows beside it).
-template <int RT, bool kDirect = false>
+template <int RT, bool kDirect = false, bool kPerScore = false>
 __device__ __forceinline__ void raw_block_staged(const AttnArgs& a, int task, int head, int split,
                                                  uint8_t* lds, int slots, int row0 = 0) {
   const int lane = threadIdx.x & 63;
@@ -592,7 +599,7 @@ __device__ __forceinline__ void raw_block_staged(const AttnArgs& a, int task, in
                                                       32 * n + 8 * wave);
       vq[e] = live[e] ? v : make_uint2(0u, 0u);
     }
-    raw_block_tail(st, sc, s, vq, pos, live, a.scale_log2, g);
+    raw_block_tail<kPerScore>(st, sc, s, vq, pos, live, a.scale_log2, g);
     if (issued < nblk) barrier_lds();  // every wavefront has read the slot refilled next
   }
   raw_finish<RT, kDirect>(a, s, head, split, st, n, g, wave);
