@@ -204,9 +204,10 @@ def prepare_tasks(qstarts, counts, tasks, task_count, max_reqs, query_tile, num_
 def step_sources_fit(query_start_loc, seq_lens, slot_mapping, block_table, num_reqs, num_tokens,
                      device):
     """Whether ``prepare_step`` reads these scheduler tensors itself: contiguous rows of the
-    buffers' own types on the buffers' own device, at least as long as the step. Any other
-    form (other types, strides or devices) is left to tensor copies, which convert."""
-    return all(
+    buffers' own types on the buffers' own device, at least as long as the step, and a request
+    and a table column to copy. Any other form (other types, strides or devices, an empty step) is
+    left to tensor copies, which convert."""
+    return num_reqs >= 1 and all(
         t.dtype == dtype and t.dim() == 1 and t.shape[0] >= need and t.device == device
         and t.stride(0) == 1
         for t, dtype, need in ((query_start_loc, torch.int32, num_reqs + 1),
@@ -214,7 +215,8 @@ def step_sources_fit(query_start_loc, seq_lens, slot_mapping, block_table, num_r
                                (slot_mapping, torch.int64, num_tokens))
     ) and (block_table.dtype == torch.int32 and block_table.dim() == 2
            and block_table.shape[0] >= num_reqs and block_table.device == device
-           and (block_table.shape[1] < 2 or block_table.stride(1) == 1)
+           and (block_table.shape[1] == 1
+                or block_table.shape[1] > 1 and block_table.stride(1) == 1)
            and block_table.stride(0) >= block_table.shape[1])
 
 

@@ -81,3 +81,18 @@ def test_other_forms_take_the_general_path():
     for i, others in forms.items():
         for other in others:
             assert not kernels.step_sources_fit(*sources[:i], other, *sources[i + 1:], 3, 8, dev)
+
+
+@pytest.mark.parametrize("requests,columns", [(0, 0), (0, 5), (2, 0)])
+def test_steps_without_requests_or_columns(requests, columns):
+    # Nothing to copy: empty tensors, which have no address.
+    b = _builder()
+    i32 = dict(dtype=torch.int32, device=DEV)
+    starts = torch.arange(requests + 1, **i32)
+    b.build(0, SimpleNamespace(
+        num_reqs=requests, num_actual_tokens=requests, max_query_len=1, query_start_loc=starts,
+        seq_lens=torch.ones(requests, **i32),
+        block_table_tensor=torch.zeros((requests, columns), **i32),
+        slot_mapping=torch.arange(requests, dtype=torch.int64, device=DEV), max_seq_len=None,
+        causal=True, attn_state=None))
+    assert b.counts.tolist() == [requests, requests] and b.task_count.item() == requests
