@@ -45,11 +45,11 @@ CONFIGS = {
     # --mode prefill only (initial prefill, no cached tokens): every token is a query token.
     "p1": dict(batch=4, context=4096, qlen=4096, ragged=False, splits="reference",
                desc="initial prefill: B4 x 4096 tokens, GQA 6:1, D256, causal"),
-    # --mode prefill: a continuation chunk over a cached prefix (one history split, the long
-    # chunk rule of config.py:86-87); the history branch is MFMA-bound.
+    # --mode prefill: a continuation chunk over a cached prefix; its history branch is split over
+    # the CUs (config.choose_chunk_splits) and bound by vector issue.
     "p2": dict(batch=1, context=32768 + 2048, qlen=2048, ragged=False, splits="device",
                desc="continuation chunk: 2048 query tokens over 32768 cached tokens, GQA 6:1, "
-                    "D256, one history split"),
+                    "D256"),
 }
 
 
@@ -574,8 +574,8 @@ def continuation_flops(w):
     """MFMA work of a continuation step: per request, the history branch (every query row
     against the request's INT2 history tokens) and the BF16 branch (the sink and recent
     window, then the chunk's own tokens causally). Useful flops count 4 per (query row, key,
-    dim): QK and PV products. The history kernel issues 6: its QK runs the query as two FP8
-    terms (hi + lo) against the FP4 codes."""
+    dim): QK and PV products. The history kernel issues 8: the query rows and the probabilities
+    enter as two FP8 terms (hi + lo) against the FP4 codes."""
     cfg = w.cfg
     hist_pairs = bf16_pairs = 0
     for prefix, hist in zip(w.prefixes, history_lengths(w)):
@@ -585,16 +585,16 @@ def continuation_flops(w):
         bf16_pairs += w.qlen * window + w.qlen * (w.qlen + 1) // 2
     per_pair = 6 * 256  # query heads x head dim
     return SimpleNamespace(history_useful=4.0 * hist_pairs * per_pair,
-                           history_issued=6.0 * hist_pairs * per_pair,
+                           history_issued=8.0 * hist_pairs * per_pair,
                            bf16=4.0 * bf16_pairs * per_pair)
 
 
 def continuation_measurement(args, w, device, name, steps):
     """A continuation chunk (config p2): the layer step as ``impl.forward`` runs it (eager
     launches: a 2048-token step is far above launch overheads), and its history branch alone,
-    timed with HIP events. The history branch is MFMA-bound: its issued FP8 x FP4 work over
-    the launch time against the FP8 dense peak (5.0 PFLOP/s, the rate of
-    v_mfma_scale_f32_16x16x128_f8f6f4 with an FP8 operand)."""
+    timed with HIP events. The history branch is matrix work, bound by the vector instructions
+    around it: its issued FP8 x FP4 work over the launch time against the FP8 dense peak (5.0
+    PFLOP/s, the rate of v_mfma_scale_f32_16x16x128_f8f6f4 with an FP8 operand)."""
     import torch
 
     from oscar_new_amd.backend import OscarAttentionImpl
@@ -621,7 +621,8 @@ def continuation_measurement(args, w, device, name, steps):
                 "kernel": bname, "us": b_us, "issued_flops": fl.history_issued,
                 "useful_flops": fl.history_useful, "tflops_issued": hist_tf,
                 "tflops_useful": fl.history_useful / (b_us * 1e-6) / 1e12,
-                "peak_tflops": 5000.0, "frac": hist_tf / 5000.0, "bound": "mfma (fp8 x fp4)"},
+                "peak_tflops": 5000.0, "frac": hist_tf / 5000.0,
+                "bound": "vector issue (mfma fp8 x fp4)"},
             "bf16_branch_flops": fl.bf16}
 
 
