@@ -20,11 +20,13 @@
 // One barrier per chunk. The wavefronts of a workgroup hold different rows, so no states are
 // merged. 150 KB of LDS, one workgroup per CU, two wavefronts per SIMD.
 //
-// What bounds it: vector issue. A chunk costs a wavefront 430 vector instructions beside its 64
-// MFMAs, and an FP8 MFMA holds the SIMD's vector issue for about 18 of its 32 cycles (measured),
-// so two wavefronts need about 6700 cycles of the 9100 a chunk takes. 2048 tokens x 6 heads over
-// 32768: 654 us (task-shaped kernel) -> 432 us with five splits; 389 tokens over 20011 beside 15
-// decodes: 254 -> 104 us.
+// What bounds it: vector issue, and the waits of a wavefront for the others of its workgroup. A
+// chunk takes a SIMD's two wavefronts 9100 cycles: their vector instructions (about 460 per
+// wavefront, beside 64 MFMAs) hold its issue for 58 % of them, the matrix pipe is busy for 45 %, and
+// a wavefront spends 38 % of its cycles at an s_waitcnt or the barrier (counters, 2048 tokens x 6
+// heads over 32768). That chunk: 654 us (task-shaped kernel, one split) -> 415 us with five splits;
+// 389 tokens over 20011 beside 15 decodes: 254 -> 102 us. Which steps take it:
+// config.chunk_kernel_pays.
 #include <type_traits>
 
 #include "dma.h"

@@ -6,9 +6,10 @@
 // 256 output dims) and streams the request's keys and values in 32-token blocks that its
 // wavefronts share: each block is copied into LDS once by direct-to-LDS loads (four stages,
 // three blocks in flight while one is computed, one barrier per block), so the K/V bytes a
-// workgroup reads from L2 serve all of its 192 rows. The copies, 32 KiB per block and
-// workgroup, are what bounds the kernel: 128-row workgroups took 16 % longer, and one block in
-// flight 11 % longer. The arithmetic of every row is the BF16 branch's (raw.h: the same MFMA
+// workgroup reads from L2 serve all of its 192 rows (128-row workgroups took 16 % longer, one block
+// in flight 11 %). What bounds it: the LDS, whose port the operand reads, the block copies and the
+// pairing of V share; the matrix pipe is busy for 47 % of the cycles, and a wavefront spends 37 % of
+// its own at an s_waitcnt or the barrier (4 prompts of 4096 tokens). The arithmetic of every row is the BF16 branch's (raw.h: the same MFMA
 // operands and k order, the same lazy max, p, sums and normalization), so the output, the LSE
 // and the bits are those of the decode path (attention_partials raw + merges) for a request
 // without history. Blocks past a workgroup's last query are not read (they are masked for

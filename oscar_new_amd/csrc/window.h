@@ -44,9 +44,13 @@ constexpr int kWindowRound = (kThreads / kWave) * kWindowBatch;  // writers of a
 
 // Workgroups per (request, kv head). A workgroup's rounds of 32 writers follow one another, each
 // a round trip to memory (about 1.5 us), so a request with many writers (a prompt: up to S + C)
-// gets one workgroup per round while the launch stays under `cap` workgroups; decode steps
-// (at most n - requests + 1 tokens in one request) keep one. Four prompts of 4096 tokens,
-// S + C = 136: one workgroup each 20.6 us; nine of up to 1201, S + C = 324, two kv heads: 32.8 us.
+// gets one workgroup per round while the launch stays under `cap` workgroups. `requests` is the
+// engine's capacity, so a full decode batch keeps one workgroup per request (a request has at most
+// n - requests + 1 tokens), a large capacity keeps few, and a workgroup without a round left reads
+// the request's lengths and ends (64 MTP requests of 4 tokens take 3 parts: post-attention 19.0 us
+// either way). Four prompts of 4096 tokens,
+// S + C = 136: one workgroup each 20.6 us, one per round 6.9; nine of up to 1201, S + C = 324, two kv
+// heads: 32.8 and 6.8 us.
 inline int window_parts(int64_t n, int64_t requests, int64_t groups, const Layout& L, int64_t cap) {
   int64_t writers = n - requests + 1;
   if (writers > L.sink + L.ring) writers = L.sink + L.ring;

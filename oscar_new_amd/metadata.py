@@ -223,11 +223,11 @@ class OscarMetadataBuilder:
         seq_cpu = getattr(cm, "seq_lens_cpu", None)
         starts_cpu = getattr(cm, "query_start_loc_cpu", None)
         total_query_keys = None
-        if not dummy and nr > 1 and cm.max_query_len > 16 and all(
+        if not (dummy or initial) and nr > 1 and cm.max_query_len > 16 and all(
                 isinstance(t, torch.Tensor) and t.device.type == "cpu" for t in (seq_cpu, starts_cpu)):
             starts = starts_cpu.numpy()[: nr + 1]
-            total_query_keys = int(((starts[1:] - starts[:-1]).astype("int64")
-                                    * seq_cpu.numpy()[:nr]).sum())
+            queries = (starts[1:] - starts[:-1]).astype("int64")
+            total_query_keys = int(queries.dot(seq_cpu.numpy()[:nr].astype("int64")))
         return OscarMetadata(
             self.qstarts, self.seqs, self.table, self.slots, self.counts, nr, nt,
             cm.max_query_len, self.max_reqs, self.layout, attn_state=state,

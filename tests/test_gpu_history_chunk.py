@@ -13,8 +13,10 @@ import pytest
 import torch
 
 from oscar_new_amd import kernels
+from oscar_new_amd.backend import OscarAttentionImpl
 from oscar_new_amd.config import OscarConfig
-from tests._state import assert_lse_close, assert_scaled_close, make_state, prepare_prefix
+from tests._state import (assert_lse_close, assert_scaled_close, make_state, native_views,
+                          prepare_prefix)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -118,7 +120,61 @@ def test_a_request_cut_short_by_the_token_count():
     _check([900, 1300], [850, 1100], 2, 6, live=171)
 
 
-def test_more_history_blocks_than_the_table_holds():
-    # 2048 kernel blocks of 128 tokens lie in LDS; 280000 tokens in one split use 2188.
-    print("[history chunk] 280000 tokens", flush=True)
-    _check([280100], [280080], 1, 6, pages=368)
+@pytest.mark.parametrize("prefix", [131200, 131201, 280080])
+def test_more_chunks_than_the_table_holds(prefix):
+    # The record offsets of 1024 chunks of 128 tokens lie in LDS; the history starts in the first
+    # chunk and ends 128 tokens before the prefix: the last chunk that fits, the next, 2188 chunks.
+    print(f"[history chunk] {prefix} tokens", flush=True)
+    _check([prefix + 20], [prefix], 1, 6, pages=(prefix + 20) // 768 + 3)
+
+
+@pytest.mark.parametrize("lengths,prefixes,hq,kv_heads", [
+    ([6100], [6000], 6, 1),  # a lone chunk, below and from 64 query tokens
+    ([6030], [6000], 6, 1),
+    ([9040, 700, 1500], [9000, 699, 1499], 8, 1),  # decodes beside it
+    ([7050, 1300], [7000, 1299], 8, 2),
+])
+def test_steps_that_take_the_tile_kernel(lengths, prefixes, hq, kv_heads):
+    """Layer steps whose host-side lengths select the kernel and several splits: the fused and the
+    single launches carry the same bits, the task-shaped kernel's step agrees within rounding."""
+    print(f"[history chunk] step {lengths} {hq}:{kv_heads}", flush=True)
+    cfg = OscarConfig(sink_tokens=4, recent_tokens=128)
+    torch.manual_seed(41)
+    layout, raw, hist, window, meta, tables = make_state(lengths, prefixes, cfg, pages=24,
+                                                         kv_heads=kv_heads)
+    rot = [torch.linalg.qr(torch.randn(256, 256))[0].bfloat16().to(DEV) for _ in range(2)]
+    ks = [torch.randn(n, kv_heads, 256).bfloat16() for n in lengths]
+    vs = [torch.randn(n, kv_heads, 256).bfloat16() for n in lengths]
+    prepare_prefix(ks, vs, *rot, hist, window, meta, tables, layout, prefixes)
+    k, v = (torch.cat([x[p:] for x, p in zip(xs, prefixes)]).to(DEV) for xs in (ks, vs))
+    n = k.shape[0]
+    q = torch.randn(n, hq, 256).bfloat16().to(DEV)
+    meta.layout, meta.num_actual_tokens = layout, n
+    meta.max_seq_len, meta.total_seq_len = max(lengths), sum(lengths)
+    meta.total_query_keys = sum((a - b) * a for a, b in zip(lengths, prefixes))
+    kernels.prepare_tasks(meta.query_start_loc, meta.counts, meta.tasks, meta.task_count,
+                          meta.max_num_reqs, cfg.queries_per_tile)
+
+    def step(fused):
+        impl = OscarAttentionImpl.standalone(hq, 256, 1 / 16, kv_heads, cfg, fused=fused)
+        impl.set_rotations(*rot)
+        splits, rule = impl.partition_for(meta)
+        name = kernels.history_kernel_name(meta, layout, hq, n, rule, splits=splits)
+        cache = raw.clone()
+        meta.merged_lse = torch.full((n, hq), 7.0, device=DEV)
+        out = torch.full((n, hq * 256), 3.0, device=DEV, dtype=torch.bfloat16)
+        impl.forward(None, q, k, v, native_views(cache, layout, 24), meta, out)
+        torch.cuda.synchronize()
+        return (out.cpu(), meta.merged_lse.cpu(), cache.cpu()), name, splits
+
+    got, name, splits = step(True)
+    assert name == "history_chunk_kernel" and splits > 1
+    for a, b in zip(got, step(False)[0]):
+        assert torch.equal(a, b)
+    meta.max_seq_len = None  # no host-side length
+    want, name, splits = step(True)
+    assert name != "history_chunk_kernel" and splits == 1
+    assert torch.equal(got[2], want[2])
+    for r in range(n):
+        assert_scaled_close(got[0][r].float().numpy(), want[0][r].float().numpy(), f"row {r}")
+    assert_lse_close(got[1].numpy(), want[1].numpy(), "merged LSE")

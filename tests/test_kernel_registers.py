@@ -1,8 +1,7 @@
 """Registers and spills of the kernels that hold the BF16 branch, from the ISA that hipcc emits (no
-GPU): the
-block-after-block form, which steps of 9 to 16 query rows per task take, is not compiled into one
-kernel with the form of few decode requests, whose 256 accumulated dims per wavefront set the
-registers of the whole kernel."""
+GPU): the block-after-block form, which steps of 9 to 16 query rows per task take, is not compiled
+into one kernel with the form of few decode requests, whose 256 accumulated dims per wavefront set
+the registers of the whole kernel; the work queue's role does not spill more scalars."""
 
 import re
 import subprocess
