@@ -630,14 +630,14 @@ def _chunk_history(meta, layout, hq, tokens, splits, split_tokens):
     query tokens in some request, more than 8 query rows per task, the reference split rule, and
     ``chunk_kernel_pays`` by the metadata's host-side request count and lengths."""
     mql = getattr(meta, "max_query_len", None)
-    longest = getattr(meta, "max_seq_len", None)
-    return (isinstance(mql, int) and mql > 16 and not split_tokens and isinstance(longest, int)
-            and history_rows(meta, layout, hq) > 8
+    if split_tokens or not isinstance(mql, int) or mql <= 16:
+        return False
+    longest, tile = getattr(meta, "max_seq_len", None), layout.config.queries_per_tile
+    return (isinstance(longest, int) and tile * (hq // layout.kv_heads) > 8
             and chunk_kernel_pays(tokens, getattr(meta, "num_reqs", meta.max_num_reqs),
                                   layout.kv_heads, hq, splits, longest,
                                   getattr(meta, "total_seq_len", None),
-                                  getattr(meta, "total_query_keys", None),
-                                  layout.config.queries_per_tile))
+                                  getattr(meta, "total_query_keys", None), tile))
 
 
 def history_kernel_name(meta, layout, hq, tokens=0, split_tokens=0, use_queue=True, splits=1):
